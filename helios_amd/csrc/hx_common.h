@@ -75,6 +75,19 @@ struct Elem<_Float16> {
 // arguments are <= 0; results below 2^-126 flush to zero and 2^-inf is 0.
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// x / (1 + e^-x) in fp32. e^-x as 2^(hi + lo) with hi + lo = -x log2(e) to twice the fp32
+// precision (the raw v_exp_f32 of a rounded product loses up to |x| ulps). -x is clamped
+// where e^-x has left fp32 either way, which keeps lo finite for infinite x; the quotient
+// then has the limits of x / (1 + e^-x), and a NaN stays one through the division.
+__device__ __forceinline__ float silu(float x) {
+  const float t = fminf(fmaxf(-x, -120.f), 120.f);
+  const float hi = __fmul_rn(t, 1.44269504f);
+  const float lo = fmaf(t, 1.92596299e-8f, fmaf(t, 1.44269504f, -hi));
+  const float e2 = fast_exp2(hi);
+  const float e = e2 < 3e38f ? fmaf(e2, __fmul_rn(lo, 0.69314718f), e2) : e2;
+  return __fdiv_rn(x, __fadd_rn(1.f, e));
+}
+
 // Two floats rounded to nearest-even and packed as {lo, hi} 16-bit elements.
 template <typename T>
 __device__ __forceinline__ uint32_t pack2_round(float lo, float hi);

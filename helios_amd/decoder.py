@@ -4,10 +4,11 @@ Mirrors Qwen3Model._forward_packed (src/helios/runtime/qwen3/model.py:92-110) an
 TransformerBlock / GroupedQueryAttention / FeedForward forwards it runs
 (layers.py:13-27, :131-164, :202-232), with random-init weights (no checkpoint is
 fetched). This is the caller of the hot path, kept to measure it in place: torch runs
-the projections, MLP and norms on hipBLASLt / elementwise kernels, and the attention
-step goes through ``PackedBatchCache.attend_projected`` (fused q/k norm + RoPE + KV
-append, then paged attention) or, with ``fused_rope=False``, through the reference's
-own sequence (torch q/k norm and RoPE, then ``attend``).
+the products on hipBLASLt, the steps between them are one launch each
+(``ops.add_rms_norm``, ``ops.swiglu``), and the attention step goes through
+``PackedBatchCache.attend_projected`` (fused q/k norm + RoPE + KV append, then paged
+attention). With ``fused_rope=False`` everything but the attention is the reference's own
+sequence of torch operations (norms, RoPE, SiLU, then ``attend``).
 
 The q, k and v projections are one GEMM over concatenated weights, and gate/up another;
 the arithmetic is otherwise the reference's.
@@ -92,8 +93,12 @@ class PagedQwen3Decoder:
         eps = config.rms_norm_eps
         x = self.embedding[input_ids]
         tokens = x.shape[1]
+        branch = None  # the last branch's output, not yet added to the residual stream
         for index, layer in enumerate(self.layers):
-            h = _rms_norm(x, layer["input_norm"], eps)
+            if fused_rope:
+                x, h = ops.add_rms_norm(x, branch, layer["input_norm"], eps)
+            else:
+                h = _rms_norm(x, layer["input_norm"], eps)
             qkv = h @ layer["qkv"].t()
             q, k, v = qkv[..., :hq], qkv[..., hq:hq + hkv], qkv[..., hq + hkv:]
             if attention_events is not None:
@@ -114,10 +119,17 @@ class PagedQwen3Decoder:
                 end.record()
                 attention_events.append((start, end))
             context = context.transpose(1, 2).reshape(1, tokens, -1)
-            x = x + context @ layer["o"].t()
+            branch = context @ layer["o"].t()
+            if fused_rope:
+                x, h = ops.add_rms_norm(x, branch, layer["post_norm"], eps)
+                branch = ops.swiglu(h @ layer["gate_up"].t()) @ layer["down"].t()
+                continue
+            x = x + branch
             h = _rms_norm(x, layer["post_norm"], eps)
             gate, up = (h @ layer["gate_up"].t()).chunk(2, dim=-1)
             x = x + (torch.nn.functional.silu(gate) * up) @ layer["down"].t()
+        if fused_rope and branch is not None:
+            x = x + branch
         cache.advance_packed()
         if greedy and fused_rope:
             return ops.final_norm_logits_argmax(x, cache.logit_indices, self.final_norm, self.embedding,

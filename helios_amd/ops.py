@@ -281,6 +281,53 @@ def attn_merge(out: torch.Tensor, lse_out: torch.Tensor, o_a: torch.Tensor, lse_
     _capi.check(code, "hx_attn_merge")
 
 
+# ------------------------------------------------- between the block's products
+def add_rms_norm(x: torch.Tensor, y: torch.Tensor | None, norm_weight: torch.Tensor,
+                 eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """``(s, RMSNorm(s))`` of ``s = x + y`` (``s = x`` without ``y``): the residual add and
+    the norm after it (layers.py:30-40, :202-232) in one launch. ``x`` / ``y`` bfloat16 or
+    float16 ``[..., hidden]`` contiguous; ``norm_weight`` ``[hidden]``, float32 (another
+    floating type is widened first)."""
+    device = _require_gpu(x, norm_weight) if y is None else _require_gpu(x, norm_weight, y)
+    dtype = _SUPPORTED.get(x.dtype)
+    if dtype is None:
+        raise ValueError("add_rms_norm supports bfloat16 and float16.")
+    if not x.is_contiguous() or x.ndim < 1 or (y is not None and (y.shape != x.shape or y.dtype != x.dtype
+                                                                 or not y.is_contiguous())):
+        raise ValueError("x and y must be contiguous, of one shape and dtype.")
+    hidden = x.shape[-1]
+    if tuple(norm_weight.shape) != (hidden,) or not norm_weight.is_floating_point():
+        raise ValueError("norm_weight must be floating-point [hidden].")
+    norm_weight = norm_weight.float().contiguous()  # no copy for the usual float32 vector
+    total = x if y is None else torch.empty_like(x)
+    normed = torch.empty_like(x)
+    if x.numel():
+        code = _capi.lib().hx_add_rms_norm(
+            x.data_ptr(), hidden, None if y is None else y.data_ptr(), hidden, norm_weight.data_ptr(), eps,
+            x.numel() // hidden, hidden, dtype, None if y is None else total.data_ptr(), normed.data_ptr(),
+            _stream_ptr(device))
+        _capi.check(code, "hx_add_rms_norm")
+    return total, normed
+
+
+def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
+    """``silu(gate) * up`` (layers.py:13-27) of ``gate_up`` ``[..., 2 * ffn]`` (gate first),
+    contiguous bfloat16 or float16; ``[..., ffn]``."""
+    device = _require_gpu(gate_up)
+    dtype = _SUPPORTED.get(gate_up.dtype)
+    if dtype is None:
+        raise ValueError("swiglu supports bfloat16 and float16.")
+    if gate_up.ndim < 1 or gate_up.shape[-1] % 2 or not gate_up.is_contiguous():
+        raise ValueError("gate_up must be contiguous [..., 2 * ffn].")
+    ffn = gate_up.shape[-1] // 2
+    out = torch.empty((*gate_up.shape[:-1], ffn), dtype=gate_up.dtype, device=device)
+    if out.numel():
+        code = _capi.lib().hx_swiglu(gate_up.data_ptr(), 2 * ffn, out.numel() // ffn, ffn, dtype, out.data_ptr(),
+                                     _stream_ptr(device))
+        _capi.check(code, "hx_swiglu")
+    return out
+
+
 # --------------------------------------------------------------- logits and argmax
 class GreedyHeads(NamedTuple):
     """Result of ``final_norm_logits_argmax``: ``token_ids`` int64 ``[n]`` (-1 for an index

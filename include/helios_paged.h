@@ -493,6 +493,21 @@ int hx_final_norm_logits_argmax(const void* hidden_states, int64_t hidden_row_st
                                 void* logits, int64_t logits_row_stride,
                                 void* workspace, size_t workspace_bytes, void* stream);
 
+/* The decoder block's steps between its products (layers.py:13-40, :202-232).
+ *
+ * hx_add_rms_norm: sum_out = x + y (rounded to the element type), norm_out =
+ * round(sum * rsqrt(mean(sum^2) + eps) * norm_weight), statistics in fp32. With y NULL
+ * there is no add, and sum_out is not written. hx_swiglu: out = silu(gate) * up, silu in
+ * fp32 and rounded before the product; a row of gate_up holds gate[ffn], then up[ffn].
+ * Strides are in elements; sum_out, norm_out and out are contiguous rows; the outputs
+ * must not overlap the inputs. Any row length; 16-byte aligned rows of a multiple of 8
+ * elements (norm: up to 8192) use 16-byte accesses. */
+int hx_add_rms_norm(const void* x, int64_t x_row_stride, const void* y, int64_t y_row_stride,
+                    const float* norm_weight, float eps, int64_t rows, int32_t hidden,
+                    int32_t dtype, void* sum_out, void* norm_out, void* stream);
+int hx_swiglu(const void* gate_up, int64_t row_stride, int64_t rows, int32_t ffn,
+              int32_t dtype, void* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
