@@ -107,8 +107,7 @@ struct Layout {
 // split count is below 2 * kChunkFillWGs / (hkv * head_quads); a block has at most
 // min(rows_per_item, max_q) rows, so that bounds the chunk partial rows. Each split adds
 // at most one item per block and head quad.
-inline Layout make_layout(int batch, int max_q, int max_k, int hq, int hkv) {
-  const Geometry geo = geometry(hq, hkv);
+inline Layout make_layout(int batch, int max_q, int max_k, int hq, int hkv, const Geometry& geo, size_t o_bytes) {
   Layout l;
   const int64_t splits = max_k > 0 ? ceil_div(max_k, kSplit) : 1;
   l.max_dec = (int64_t)batch * splits;
@@ -129,9 +128,14 @@ inline Layout make_layout(int batch, int max_q, int max_k, int hq, int hkv) {
   l.pf_seq = off;    off = align256(off + (size_t)l.max_pf * sizeof(int4));
   const int64_t slots = l.max_dec + l.cslot_cap;
   l.part_ml = off;   off = align256(off + (size_t)slots * hq * sizeof(float2));
-  l.part_o = off;    off = align256(off + (size_t)slots * hq * kD * sizeof(uint16_t));
+  l.part_o = off;    off = align256(off + (size_t)slots * hq * o_bytes);
   l.total = off;
   return l;
+}
+// Of the decode / chunk kernels: 16-bit partial rows of kD elements. Also the size every
+// workspace must have, whichever kernels serve its shape.
+inline Layout make_layout(int batch, int max_q, int max_k, int hq, int hkv) {
+  return make_layout(batch, max_q, max_k, hq, hkv, geometry(hq, hkv), kD * sizeof(uint16_t));
 }
 
 // Key tiles [*tb, *te) of the chunk row block starting at row0 (rows_per_item rows) of a
@@ -266,6 +270,8 @@ struct PlanArgs {
   int32_t rows_per_item, head_quads;
   int32_t win_left, win_right;
   int32_t hq, hkv;
+  int32_t stamp;
+  int32_t plain;  // sequence info only, no work lists
 };
 
 __device__ int block_exclusive_scan(int v, int* wave_tot, int* total) {
@@ -352,7 +358,7 @@ __device__ void write_plan_header(const PlanArgs& a, int err, int4 totals) {
   a.hdr[H_MAXK] = a.max_k;
   a.hdr[H_HQ] = a.hq;
   a.hdr[H_HKV] = a.hkv;
-  a.hdr[H_STAMP] = kPlanStamp;
+  a.hdr[H_STAMP] = a.stamp;
 }
 
 // The planner's serial form: one thread walks each sequence's row blocks in every pass.
@@ -600,6 +606,17 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
     best_one = INT32_MAX;
   }
   int err = 0;
+  if (a.plain) {
+    __syncthreads();
+    for (int b = tid; b < a.batch; b += kPlanThreads) {
+      const SeqMeta m = plan_seq(a, b, err);
+      a.seq_info[b] = make_int4(m.q0, m.n, m.L, m.kvb);
+    }
+    if (err) atomicOr(&err_bits, err);
+    __syncthreads();
+    if (tid == 0) write_plan_header(a, err_bits, make_int4(0, 0, 0, 0));
+    return;
+  }
   int turn = 0;  // WaveTotals buffer of the next block-wide scan
 
   // Phase 0: list the chunk sequences and count their row blocks. A batch of one round
@@ -2117,177 +2134,494 @@ __global__ __launch_bounds__(kChunkThreads, 2) void chunk_pair_kernel(RunArgs a0
 }
 
 // ------------------------------------------------------------------ any head_dim
-// Attention for shapes the tuned kernels do not cover: head_dim any multiple of 8 up to
-// 256, and any group size G. One workgroup per (sequence, block of query rows, KV head
-// g, block of up to kGenUnits of g's query heads); its (row, head) units share every K/V
-// tile read. Keys go through LDS kGenTile at a time. Lane j scores key j of the tile for
-// each of its wave's units, the softmax runs online per unit in fp32, and lane j
-// accumulates O for dims j, j + 64, ... of every unit, reading each key's p from LDS.
-// Decode and chunk rows alike, with no split-K: head_dim 128 with G in {1, 2, 4, 8}
-// goes to the decode / chunk kernels instead.
-constexpr int kGenUnits = 16;    // (row, head) units per workgroup, 4 per wave
-constexpr int kGenTile = 64;     // keys per LDS tile: one per lane
+// Attention for the shapes the kernels above do not cover: head_dim any multiple of 8 up
+// to 256, any group size G. The (row, head) pairs that share a KV head are flattened into
+// units, 16 to a wave, and both products run on 16x16x32 MFMA: S^T = K Q^T and
+// O^T = V^T P^T, over 64-key tiles of K and V staged in LDS by the whole workgroup (the
+// next tile's loads in flight in registers meanwhile).
+//   A block of chunk rows has up to 64 units: wave w takes units 16w .. 16w + 15 over
+//   every key of a tile.
+//   A decode row has up to 16 (a head block of its group): all four waves take the same
+//   units, wave w over keys 16w .. 16w + 15 of each tile, and merge through LDS at the end.
+// Work comes from the plan's lists: decode rows in 256-key splits, chunk blocks split over
+// their key tiles like the tuned kernels' when they would not fill the GPU. The launch is
+// persistent (kWideWGs workgroups walk the lists), since the item counts are known on the
+// device only.
+// P keeps fp32's accuracy: it goes into P V as two MFMA operands, its rounding to the
+// element type and the remainder (17 bits or more of p), and the splits' partial results
+// stay in fp32. q . k is exact products in fp32 sums.
+// Bound by latency at these sizes. 24 decode rows of 200-2048 keys and chunks of 512 and
+// 333 rows, 16/4 heads, d = 64: 19.5 us and 4.8 us for the merge; scores and P V on the VALU,
+// 16 units a workgroup and no splits, took 284 us.
+constexpr int kWideUnits = 64;   // units of a chunk block: 4 waves x 16
+constexpr int kWideDecUnits = 16;
+constexpr int kWideThreads = 256;
+constexpr int kWideWGs = 1024;   // persistent workgroups: 4 per CU
 
-struct GenericShape {
-  int32_t head_dim, group, heads_per_item, rows_per_item, row_blocks, head_blocks;
-};
-
-inline GenericShape generic_shape(int max_q, int G, int head_dim) {
-  GenericShape g;
-  g.head_dim = head_dim;
-  g.group = G;
-  g.heads_per_item = G < kGenUnits ? G : kGenUnits;
-  g.rows_per_item = kGenUnits / g.heads_per_item;
-  g.row_blocks = (int)ceil_div(max_q > 0 ? max_q : 1, g.rows_per_item);
-  g.head_blocks = (int)ceil_div(G, g.heads_per_item);
+// Chunk blocks: whole groups of query heads per row while they fit kWideUnits.
+inline Geometry wide_geometry(int hq, int hkv) {
+  Geometry g;
+  g.G = hq / hkv;
+  g.Gw = g.G < kWideUnits ? g.G : kWideUnits;
+  g.R = 1;
+  g.head_quads = (int)ceil_div(g.G, g.Gw);
+  g.rows_per_item = kWideUnits / g.Gw;
   return g;
 }
 
-template <typename T, int DMAX>
-__global__ __launch_bounds__(256) void generic_kernel(RunArgs a, GenericShape gs) {
+struct WideShape {
+  int32_t head_dim, group;
+  int32_t heads, rows;        // query heads and rows of a chunk block, at most
+  int32_t head_blocks;        // chunk blocks over a group's heads
+  int32_t dec_head_blocks;    // decode items over a group's heads
+  int32_t row_blocks;         // without lists: blocks of `rows` rows per sequence
+  int32_t lists;              // the run's workspace holds work lists and partials
+  int32_t stamp;              // wide_stamp(head_dim)
+  int64_t max_pf, max_comb;
+};
+
+// Stamp of a plan for these kernels without work lists; with them, one more. The lists and
+// the partial slots depend on head_dim.
+inline int32_t wide_stamp(int head_dim) { return kPlanStamp + 2 * head_dim; }
+
+// A plan for these kernels without lists: sequence info alone. For workspaces that hold the
+// 16-bit partials of make_layout but not the fp32 ones of wide_layout.
+inline Layout wide_plain_layout(int batch) {
+  Layout l{};
+  l.seq_info = align256(H_WORDS * sizeof(int32_t));
+  l.total = align256(l.seq_info + (size_t)batch * sizeof(int4));
+  l.dec_items = l.comb_seqs = l.pf_items = l.pf_base = l.pf_seq = l.part_ml = l.part_o = l.total;
+  return l;
+}
+
+template <typename T>
+constexpr float wide_p_shift() {  // p is scaled by 2^shift: fp16's remainders stay normal
+  return std::is_same<T, _Float16>::value ? 12.f : 0.f;
+}
+
+struct WideItem {
+  int b, q0, n, L, kvb;  // the sequence
+  int row0, rows;        // query rows [row0, row0 + rows)
+  int h0, hcount;        // query heads g * G + [h0, h0 + hcount)
+  int k_begin, k_end;    // keys this item covers
+  int64_t slot0;         // partial slot of row row0 (slots: `splits` apart), splits > 1
+  int splits;
+};
+
+template <int DP>
+struct WideLds {
+  static constexpr int kKRow = 2 * DP + 16;  // an odd number of 16-byte pieces: 16 rows' fragment reads hit 16 bank groups
+  static constexpr int kVRow = 2 * DP + 32;  // 8 rows' 32-byte transposing reads hit 8 bank groups
+  union {
+    struct {
+      __attribute__((aligned(16))) uint8_t k[kTile * kKRow];
+      __attribute__((aligned(16))) uint8_t v[kTile * kVRow];
+    } tile;
+    __attribute__((aligned(16))) float o[4][kWideDecUnits][DP];  // the waves' results of a decode item
+  };
+  float m[4][kWideDecUnits], l[4][kWideDecUnits];
+};
+
+template <typename T, int DP, bool DEC>
+__device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws, WideLds<DP>& lds, const int g,
+                                          const WideItem& it) {
   typedef hx::Elem<T> E;
-  constexpr int KS = DMAX + 8;                      // K tile row stride (elements)
-  constexpr int NC = DMAX >= 64 ? DMAX / 64 : 1;    // O dims per lane and unit
-  __shared__ __attribute__((aligned(16))) T k_lds[kGenTile * KS];
-  __shared__ __attribute__((aligned(16))) T v_lds[kGenTile * DMAX];
-  __shared__ __attribute__((aligned(16))) float q_lds[kGenUnits * DMAX];
-  __shared__ float p_lds[kGenUnits][kGenTile];
+  constexpr int kPieces = DP / 8;                       // 16-byte pieces of a padded row
+  constexpr int NP = kTile * kPieces / kWideThreads;    // pieces per thread and tile, K and V each
+  constexpr int NS = DP / 32, NO = DP / 16;             // QK^T steps, O blocks
+  constexpr int NB = DEC ? 1 : 4;                       // 16-key blocks of a tile a wave takes
+  constexpr int NK = DEC ? 1 : 2;                       // P V key steps per tile
+  const int tid = hx::tid_x(), lane = tid & 63, gg = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int D = ws.head_dim;
+  const int units = it.rows * it.hcount;
+  const int u0 = DEC ? 0 : 16 * w;
+  const int u = u0 + (lane & 15);
+  const bool unit_ok = u < units;
+  const int urow = unit_ok ? u / it.hcount : 0;
+  const int qh = g * ws.group + it.h0 + (unit_ok ? u - urow * it.hcount : 0);
+  const int qpos = it.L - it.n + it.row0 + urow;
+  const bool busy = u0 < units;  // wave-uniform
 
-  const int tid = hx::tid_x(), lane = tid & 63, w = tid >> 6;
-  const int D = gs.head_dim;
-  int x = hx::wg_x();
-  const int hb = x % gs.head_blocks;
-  x /= gs.head_blocks;
-  const int g = x % a.hkv;
-  x /= a.hkv;
-  const int rb = x % gs.row_blocks;
-  const int b = x / gs.row_blocks;
-  const Header hd = read_header(a);
-  if (!hd.ok || b >= a.batch) return;
-  const int4 si = a.seq_info[b];
-  const int q0 = si.x, n = si.y, L = si.z, kvb = si.w;
-  const int row0 = rb * gs.rows_per_item;
-  if (row0 >= n) return;
-  const int rows = min(gs.rows_per_item, n - row0);
-  const int h0 = hb * gs.heads_per_item;
-  const int hcount = min(gs.heads_per_item, gs.group - h0);
-  const int units = rows * hcount;  // unit u: row row0 + u / hcount, head g*G + h0 + u % hcount
-
-  // The units' queries, widened to fp32.
-  for (int idx = tid; idx < units * D; idx += 256) {
-    const int u = idx / D, d = idx - (idx / D) * D;
-    const int64_t qrow = query_row(a, q0 + row0 + u / hcount);
-    const int qh = g * gs.group + h0 + u % hcount;
-    q_lds[u * DMAX + d] = E::lo(reinterpret_cast<const uint16_t*>(a.q)[qrow * a.q_row + (int64_t)qh * a.q_head + d]);
-  }
-  // Keys any row of the block can see: [klo, khi].
-  const int qfirst = L - n + row0, qlast = L - n + row0 + rows - 1;
-  const int klo = a.win_left >= 0 ? max(0, qfirst - a.win_left) : 0;
-  int khi = L - 1;
-  if (a.win_right >= 0) khi = min(khi, qlast + a.win_right);
-
-  float m[4], l[4], o[4][NC];
+  // Q^T as the MFMA B operand: lane holds its unit's dims 32st + 8(lane>>4)..+7.
+  uint4 qf[NS];
+  {
+    const T* qp = reinterpret_cast<const T*>(a.q) + query_row(a, it.q0 + it.row0 + urow) * a.q_row +
+                  (int64_t)qh * a.q_head + 8 * gg;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    m[k] = -INFINITY;
-    l[k] = 0.f;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) o[k][c] = 0.f;
+    for (int st = 0; st < NS; ++st) qf[st] = unit_ok && 32 * st + 8 * gg < D ? ld16(qp + 32 * st) : hx::zero4();
   }
-  const int chunks = D / 8;  // 16-byte pieces of a head row
-  const T* kbase = reinterpret_cast<const T*>(a.k) + (int64_t)g * a.kv_head;
-  const T* vbase = reinterpret_cast<const T*>(a.v) + (int64_t)g * a.kv_head;
-  for (int t0 = khi >= klo ? (klo / kGenTile) * kGenTile : 0; khi >= klo && t0 <= khi; t0 += kGenTile) {
-    __syncthreads();  // the previous tile's readers are done
-    // K and V rows of keys t0 .. t0 + 63; keys past L - 1 re-read row L - 1 (masked).
-    for (int idx = tid; idx < kGenTile * chunks; idx += 256) {
-      const int key = idx / chunks, c8 = idx - (idx / chunks) * chunks;
-      const int kk = min(t0 + key, L - 1);
-      int64_t row;
-      if (a.page_size > 0) {
-        int page = a.bt[(int64_t)b * a.bt_stride + kk / a.page_size];
-        if ((unsigned)page >= (unsigned)a.num_pages) {
-          atomicOr(&a.hdr[H_ERR], HX_WERR_BAD_PAGE);
-          page = 0;
-        }
-        row = (int64_t)page * a.page_size + kk % a.page_size;
-      } else {
-        row = (int64_t)kvb + kk;
+  // Keys the unit sees within this item.
+  int klo = it.k_begin, khi = it.k_end - 1;
+  if (a.win_left >= 0) klo = max(klo, qpos - a.win_left);
+  if (a.win_right >= 0) khi = min(khi, qpos + a.win_right);
+  khi = unit_ok ? khi : -1;
+
+  const int t_begin = it.k_begin / kTile, t_end = it.k_end > it.k_begin ? (it.k_end + kTile - 1) / kTile : it.k_begin / kTile;
+  // Page ids, 64 at a time: lane j holds the id of page pg_base + j.
+  const bool paged = a.page_size > 0;
+  const int last_pg = paged && t_end > t_begin ? (it.k_end - 1) / a.page_size : -1;
+  int pg_base = paged ? t_begin * kTile / a.page_size : 0, pg_ids = -1;
+  auto fetch_pages = [&]() {
+    const int p = pg_base + lane;
+    pg_ids = p <= last_pg ? a.bt[(int64_t)it.b * a.bt_stride + p] : -1;
+  };
+  if (paged && t_end > t_begin) fetch_pages();
+  bool bad_page = false;
+
+  // Thread's pieces of a tile: row and byte offset from the tile's first row of head g.
+  // Pieces past head_dim get an offset no tile reaches, which reads zeros.
+  const uint32_t row_bytes = (uint32_t)a.kv_row * (uint32_t)sizeof(T);
+  uint32_t offs[NP];
+  int k_at[NP], v_at[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    const int p = tid + j * kWideThreads, r = p / kPieces, c = p - r * kPieces;
+    offs[j] = 8 * c < D ? (uint32_t)r * row_bytes + 16u * (uint32_t)c : 0xFFFFFF00u;
+    k_at[j] = r * WideLds<DP>::kKRow + 16 * c;
+    v_at[j] = r * WideLds<DP>::kVRow + 16 * c;
+  }
+  uint4 kreg[NP], vreg[NP];
+  auto load_tile = [&](int t) {
+    const int key0 = t * kTile;
+    int64_t row = (int64_t)it.kvb + key0;
+    if (paged) {
+      const int pg = key0 / a.page_size;
+      if (pg - pg_base >= 64) {
+        pg_base = pg;
+        fetch_pages();
       }
-      *reinterpret_cast<uint4*>(&k_lds[key * KS + 8 * c8]) = ld16(kbase + row * a.kv_row + 8 * c8);
-      *reinterpret_cast<uint4*>(&v_lds[key * DMAX + 8 * c8]) = ld16(vbase + row * a.kv_row + 8 * c8);
+      int page = __builtin_amdgcn_readlane(pg_ids, pg - pg_base);
+      const bool bad = (unsigned)page >= (unsigned)a.num_pages;
+      bad_page |= bad;
+      page = bad ? 0 : page;
+      row = (int64_t)page * a.page_size + (key0 - pg * a.page_size);
     }
+    const int64_t head0 = row * a.kv_row + (int64_t)g * a.kv_head;
+    // The resources end with the last key's head row: keys past it arrive as zeros.
+    const int rows = min(it.L - key0, kTile);
+    const uint32_t range = (uint32_t)(rows - 1) * row_bytes + (uint32_t)D * (uint32_t)sizeof(T);
+    const __amdgpu_buffer_rsrc_t kres = hx::buffer_rsrc(reinterpret_cast<const T*>(a.k) + head0, range);
+    const __amdgpu_buffer_rsrc_t vres = hx::buffer_rsrc(reinterpret_cast<const T*>(a.v) + head0, range);
+#pragma unroll
+    for (int j = 0; j < NP; ++j) kreg[j] = hx::ld16_buf(kres, offs[j]);
+#pragma unroll
+    for (int j = 0; j < NP; ++j) vreg[j] = hx::ld16_buf(vres, offs[j]);
+  };
+
+  float m = -INFINITY, l = 0.f;  // running max (log2 units) of the unit; this lane's share of its sum
+  hx::f32x4_t oacc[NO];
+#pragma unroll
+  for (int db = 0; db < NO; ++db) oacc[db] = hx::f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  if (t_begin < t_end) load_tile(t_begin);
+  for (int t = t_begin; t < t_end; ++t) {
+    __syncthreads();  // the previous tile's (and item's) readers are done
+#pragma unroll
+    for (int j = 0; j < NP; ++j) *reinterpret_cast<uint4*>(lds.tile.k + k_at[j]) = kreg[j];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) *reinterpret_cast<uint4*>(lds.tile.v + v_at[j]) = vreg[j];
     __syncthreads();
-    // Scores and online softmax: lane j holds key t0 + j of each of the wave's units.
-    const int kk = t0 + lane;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int c8 = 0; c8 < chunks; ++c8) {
-      const uint4 kv = *reinterpret_cast<const uint4*>(&k_lds[lane * KS + 8 * c8]);
-      const float kf[8] = {E::lo(kv.x), E::hi(kv.x), E::lo(kv.y), E::hi(kv.y),
-                           E::lo(kv.z), E::hi(kv.z), E::lo(kv.w), E::hi(kv.w)};
+    if (t + 1 < t_end) load_tile(t + 1);
+    if (!busy) continue;
+
+    // S^T: lane holds keys 16kb + 4(lane>>4) + i of unit lane & 15 (decode: kb is the wave).
+    hx::f32x4_t s[NB];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int u = w + 4 * k;
-        if (u < units) {
-          const float4 qa = *reinterpret_cast<const float4*>(&q_lds[u * DMAX + 8 * c8]);
-          const float4 qb = *reinterpret_cast<const float4*>(&q_lds[u * DMAX + 8 * c8 + 4]);
-          s[k] += qa.x * kf[0] + qa.y * kf[1] + qa.z * kf[2] + qa.w * kf[3] +
-                  qb.x * kf[4] + qb.y * kf[5] + qb.z * kf[6] + qb.w * kf[7];
-        }
+    for (int kb = 0; kb < NB; ++kb) s[kb] = hx::f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < NS; ++st)
+#pragma unroll
+      for (int kb = 0; kb < NB; ++kb) {
+        const int kr = 16 * (DEC ? w : kb) + (lane & 15);
+        const uint4 kf = *reinterpret_cast<const uint4*>(lds.tile.k + kr * WideLds<DP>::kKRow + 16 * (4 * st + gg));
+        s[kb] = E::mfma16x16x32(hx::as_v8<T>(kf), hx::as_v8<T>(qf[st]), s[kb]);
+      }
+    const int key_base = t * kTile + (DEC ? 16 * w : 0) + 4 * gg;  // of s[0][0]
+    float mt = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = key_base + 16 * kb + i;
+        const float x = key >= klo && key <= khi ? s[kb][i] * a.scale_log2 : -INFINITY;
+        s[kb][i] = x;
+        mt = fmaxf(mt, x);
+      }
+    mt = fmaxf(m, hx::max_xor32(hx::max_xor16(mt)));
+    if (__any(mt > m)) {
+      const float alpha = m == -INFINITY ? 0.f : hx::fast_exp2(m - mt);  // nothing summed yet: any factor will do
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < NO; ++db) oacc[db] *= alpha;
+      m = mt;
+    }
+    const float neg_m = m == -INFINITY ? 0.f : wide_p_shift<T>() - m;
+    uint4 ph[NK], pl[NK];
+#pragma unroll
+    for (int kb = 0; kb < NB; ++kb) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[kb][i] = hx::fast_exp2(s[kb][i] + neg_m);  // -inf -> 0
+        l += s[kb][i];
       }
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int u = w + 4 * k;
-      if (u >= units) continue;  // wave-uniform
-      const int qpos = L - n + row0 + u / hcount;
-      const bool vis = kk <= L - 1 && (a.win_left < 0 || kk >= qpos - a.win_left) &&
-                       (a.win_right < 0 || kk <= qpos + a.win_right);
-      const float sc = vis ? s[k] * a.scale_log2 : -INFINITY;
-      const float m_new = fmaxf(m[k], wave_max(sc));
-      float p = 0.f, alpha = 1.f;
-      if (m_new != -INFINITY) {
-        p = vis ? hx::fast_exp2(sc - m_new) : 0.f;
-        alpha = m[k] == -INFINITY ? 0.f : hx::fast_exp2(m[k] - m_new);
+    for (int ks = 0; ks < NK; ++ks) {
+      uint32_t hi[4] = {0u, 0u, 0u, 0u}, lo[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < (DEC ? 2 : 4); ++j) {
+        const float x = s[DEC ? 0 : 2 * ks + (j >> 1)][2 * (j & 1)], y = s[DEC ? 0 : 2 * ks + (j >> 1)][2 * (j & 1) + 1];
+        hi[j] = hx::pack2_round<T>(x, y);
+        lo[j] = hx::pack2_round<T>(x - E::lo(hi[j]), y - E::hi(hi[j]));
       }
-      l[k] = l[k] * alpha + wave_sum(p);
-      m[k] = m_new;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) o[k][c] *= alpha;
-      p_lds[u][lane] = p;
+      ph[ks] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+      pl[ks] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
     }
-    __syncthreads();
-    // O += P V: lane owns dims lane + 64c.
+    // V^T operands, read transposed: keys {r0 + 0..3, r0 + 16 + 0..3} of dim 16db + j per
+    // lane (chunk_body's read_v); a decode wave's 16 keys fill the first half only.
+    const int i16 = lane & 15;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int u = w + 4 * k;
-      if (u >= units) continue;
-      for (int j = 0; j < kGenTile; ++j) {
-        const float pj = p_lds[u][j];
+    for (int ks = 0; ks < NK; ++ks) {
+      const int r0 = (DEC ? 16 * w : 32 * ks) + 4 * gg + (i16 >> 2);
+      const uint8_t* vp = lds.tile.v + r0 * WideLds<DP>::kVRow + 8 * (i16 & 3);
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          const int d = lane + 64 * c;
-          if (d < D) o[k][c] = fmaf(pj, E::lo(reinterpret_cast<const uint16_t*>(v_lds)[j * DMAX + d]), o[k][c]);
-        }
+      for (int db = 0; db < NO; ++db) {
+        const uint2 lo = hx::ld8_lds_tr16(vp + 32 * db);
+        const uint2 hi = DEC ? make_uint2(0u, 0u) : hx::ld8_lds_tr16(vp + 16 * WideLds<DP>::kVRow + 32 * db);
+        const uint4 vf = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        oacc[db] = E::mfma16x16x32(hx::as_v8<T>(vf), hx::as_v8<T>(ph[ks]), oacc[db]);
+        oacc[db] = E::mfma16x16x32(hx::as_v8<T>(vf), hx::as_v8<T>(pl[ks]), oacc[db]);
       }
     }
   }
-  // Normalise and store every unit of this wave.
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int u = w + 4 * k;
-    if (u >= units) continue;
-    const int64_t orow = q0 + row0 + u / hcount;
-    const int qh = g * gs.group + h0 + u % hcount;
-    const float inv = l[k] > 0.f ? 1.f / l[k] : 0.f;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int d = lane + 64 * c;
-      if (d < D)
-        reinterpret_cast<uint16_t*>(a.out)[orow * a.o_row + (int64_t)qh * a.o_head + d] = E::bits(o[k][c] * inv);
+  if (bad_page && tid == 0) atomicOr(&a.hdr[H_ERR], HX_WERR_BAD_PAGE);
+  l = hx::add_xor32(hx::add_xor16(l));
+
+  float* const part_o = reinterpret_cast<float*>(a.part_o);
+  // Result (acc / l, four dims from d0) of one unit: output row piece, or partial.
+  auto store = [&](int row, int head, int d0, float ml, float ll, const float (&x)[4]) {
+    if (it.splits > 1) {
+      const int64_t slot = it.slot0 + (int64_t)row * it.splits;
+      if (slot >= a.slot_cap) return;
+      *reinterpret_cast<float4*>(part_o + (slot * a.hq + head) * D + d0) = make_float4(x[0], x[1], x[2], x[3]);
+      if (d0 == 0) a.part_ml[slot * a.hq + head] = make_float2(ml, ll);
+      return;
     }
-    if (a.lse && lane == 0)
-      a.lse[(int64_t)qh * a.total_q + orow] = l[k] > 0.f ? (m[k] + log2f(l[k])) * kLn2 : -INFINITY;
+    const float inv = ll > 0.f ? 1.f / ll : 0.f;
+    const int64_t orow = it.q0 + it.row0 + row;
+    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + orow * a.o_row + (int64_t)head * a.o_head + d0) =
+        make_uint2(hx::pack2_round<T>(x[0] * inv, x[1] * inv), hx::pack2_round<T>(x[2] * inv, x[3] * inv));
+    if (a.lse && d0 == 0)
+      a.lse[(int64_t)head * a.total_q + orow] = ll > 0.f ? (ml + (log2f(ll) - wide_p_shift<T>())) * kLn2 : -INFINITY;
+  };
+  if constexpr (DEC) {
+    __syncthreads();  // the last tile's readers are done
+    if (gg == 0) {
+      lds.m[w][lane & 15] = m;
+      lds.l[w][lane & 15] = l;
+    }
+#pragma unroll
+    for (int db = 0; db < NO; ++db)
+      *reinterpret_cast<float4*>(&lds.o[w][lane & 15][16 * db + 4 * gg]) =
+          make_float4(oacc[db][0], oacc[db][1], oacc[db][2], oacc[db][3]);
+    __syncthreads();
+    const int quads = D / 4;
+    for (int i = tid; i < it.hcount * quads; i += kWideThreads) {
+      const int h = i / quads, d0 = 4 * (i - h * quads);
+      float mm = -INFINITY, ll = 0.f, x[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) mm = fmaxf(mm, lds.m[ww][h]);
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) {
+        const float mw = lds.m[ww][h];
+        const float alpha = mw == -INFINITY ? 0.f : hx::fast_exp2(mw - mm);
+        const float4 o4 = *reinterpret_cast<const float4*>(&lds.o[ww][h][d0]);
+        ll = fmaf(alpha, lds.l[ww][h], ll);
+        x[0] = fmaf(alpha, o4.x, x[0]);
+        x[1] = fmaf(alpha, o4.y, x[1]);
+        x[2] = fmaf(alpha, o4.z, x[2]);
+        x[3] = fmaf(alpha, o4.w, x[3]);
+      }
+      store(0, g * ws.group + it.h0 + h, d0, mm, ll, x);
+    }
+  } else {
+#pragma unroll
+    for (int db = 0; db < NO; ++db) {
+      const int d0 = 16 * db + 4 * gg;
+      const float x[4] = {oacc[db][0], oacc[db][1], oacc[db][2], oacc[db][3]};
+      if (unit_ok && d0 < D) store(urow, qh, d0, m, l, x);
+    }
+  }
+}
+
+// A work-list entry, the same for the whole workgroup: kept in scalar registers.
+__device__ __forceinline__ int4 uniform4(const int4* p) {
+  const int4 v = *p;
+  return make_int4(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y),
+                   __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w));
+}
+
+// x = q * d + r for 0 <= x, d > 0: the quotient, leaving r in x. 32-bit division unless x needs more.
+__device__ __forceinline__ int64_t split_off(int64_t& x, int d) {
+  const int64_t q = (x >> 32) == 0 ? (int64_t)((uint32_t)x / (uint32_t)d) : x / d;
+  x -= q * d;
+  return q;
+}
+
+// The plan's header, and whether its work lists are to be used: a plan and a run that were
+// given different sizes of the workspace agree on the sequence info, which is at the same
+// place with and without lists, so either alone makes every block whole.
+__device__ __forceinline__ bool wide_plan_ok(const RunArgs& a, const WideShape& ws, int4* counts, bool* lists) {
+  const int4 h0 = *reinterpret_cast<const int4*>(a.hdr);
+  const int4 h1 = *reinterpret_cast<const int4*>(a.hdr + 4);
+  const int2 h2 = *reinterpret_cast<const int2*>(a.hdr + 8);
+  *counts = h0;
+  *lists = ws.lists && h2.y == ws.stamp + 1;
+  const bool ok = ((h2.y == ws.stamp) | (h2.y == ws.stamp + 1)) & (h1.x == a.batch) & (h1.y == a.max_q) & (h1.z == a.max_k) & (h1.w == a.hq) &
+                  (h2.x == a.hkv);
+  if (!ok && hx::wg_x() == 0 && hx::tid_x() == 0) atomicOr(&a.hdr[H_ERR], HX_WERR_PLAN_MISMATCH);
+  return ok;
+}
+
+// Workgroups: n_wg of them (the launch's count). Every loop bound comes from the plan
+// header and is the same for the whole workgroup.
+template <typename T, int DP>
+__global__ __launch_bounds__(kWideThreads, DP <= 64 ? 4 : DP <= 128 ? 2 : 1) void wide_kernel(RunArgs a, WideShape ws, int n_wg) {
+  __shared__ WideLds<DP> lds;
+  int4 counts;
+  bool lists;
+  if (!wide_plan_ok(a, ws, &counts, &lists)) return;
+  const int64_t pf_work = lists ? min((int64_t)counts.y, ws.max_pf) * a.hkv : 0;
+  const int64_t dec_work = lists ? min((int64_t)counts.x, a.dec_cap) * ws.dec_head_blocks * a.hkv : 0;
+  const int64_t plain_work = lists ? 0 : (int64_t)a.batch * ws.row_blocks * ws.head_blocks * a.hkv;
+  // The chunk items first: they are the longest, listed longest first.
+  for (int64_t i = hx::wg_x(); i < pf_work + dec_work + plain_work; i += n_wg) {
+    WideItem it;
+    int64_t x = i;
+    bool decode = false;
+    int g, hb;
+    if (i < pf_work) {
+      const int64_t item = split_off(x, a.hkv);
+      g = (int)x;
+      const int4 pi = uniform4(a.pf_items + item), si = uniform4(a.pf_seq + item);
+      it.b = pi.x; it.row0 = pi.y; hb = pi.z;
+      it.q0 = si.x; it.n = si.y; it.L = si.z; it.kvb = si.w;
+      const int sp = pi.w & 0xffff;
+      it.splits = (pi.w >> 16) + 1;
+      it.slot0 = a.dec_cap + __builtin_amdgcn_readfirstlane(a.pf_base[item]) + sp;
+      it.rows = min(ws.rows, it.n - it.row0);
+      int tb, te;
+      chunk_tiles(it.n, it.L, it.row0, ws.rows, a.win_left, a.win_right, &tb, &te);
+      const int span = (te - tb + it.splits - 1) / it.splits;
+      tb = min(te, tb + sp * span);
+      te = min(te, tb + span);
+      it.k_begin = tb * kTile;
+      it.k_end = min(it.L, te * kTile);
+    } else if (i < pf_work + dec_work) {
+      x -= pf_work;
+      int64_t rest = split_off(x, a.hkv);
+      g = (int)x;
+      const int64_t item = split_off(rest, ws.dec_head_blocks);
+      hb = (int)rest;
+      const int4 di = uniform4(a.dec_items + item);  // {b, split, q0, L}
+      decode = true;
+      it.b = di.x; it.q0 = di.z; it.n = 1; it.L = di.w; it.row0 = 0; it.rows = 1;
+      it.kvb = (unsigned)it.b < (unsigned)a.batch ? uniform4(a.seq_info + it.b).w : 0;
+      int first;
+      decode_splits(it.L, a.win_left, &first, &it.splits);
+      it.slot0 = item;
+      it.k_begin = max(di.y * kSplit, decode_lo(it.L, a.win_left));
+      it.k_end = min(it.L, (di.y + 1) * kSplit);
+    } else {
+      int64_t rest = split_off(x, a.hkv);
+      g = (int)x;
+      int64_t block = split_off(rest, ws.head_blocks);
+      hb = (int)rest;
+      it.b = (int)split_off(block, ws.row_blocks);
+      const int rb = (int)block;
+      const int4 si = uniform4(a.seq_info + it.b);
+      it.q0 = si.x; it.n = si.y; it.L = si.z; it.kvb = si.w;
+      it.row0 = rb * ws.rows;
+      it.rows = min(ws.rows, it.n - it.row0);
+      it.splits = 1;
+      it.slot0 = 0;
+      int tb, te;
+      chunk_tiles(it.n, it.L, it.row0, ws.rows, a.win_left, a.win_right, &tb, &te);
+      it.k_begin = tb * kTile;
+      it.k_end = min(it.L, te * kTile);
+    }
+    if ((unsigned)it.b >= (unsigned)a.batch || it.rows < 1) continue;  // workgroup-uniform
+    const int per = decode ? kWideDecUnits : ws.heads;
+    it.h0 = hb * per;
+    it.hcount = min(per, ws.group - it.h0);
+    if (it.hcount < 1) continue;
+    if (decode) wide_item<T, DP, true>(a, ws, lds, g, it);
+    else wide_item<T, DP, false>(a, ws, lds, g, it);
+  }
+}
+
+// Merges the fp32 partials of split rows: the plan's combine records {b, first slot,
+// splits | (rows - 1) << 24, first output row} x KV heads, a thread per (row, head, four
+// dims), in split order.
+template <typename T>
+__global__ __launch_bounds__(kWideThreads) void wide_combine_kernel(RunArgs a, WideShape ws, int n_wg) {
+  int4 counts;
+  bool lists;
+  if (!wide_plan_ok(a, ws, &counts, &lists) || !lists) return;
+  const int D = ws.head_dim, quads = D / 4, per_row = ws.group * quads;
+  const float* const part_o = reinterpret_cast<const float*>(a.part_o);
+  const int64_t work = min((int64_t)counts.z, ws.max_comb) * a.hkv;
+  for (int64_t i = hx::wg_x(); i < work; i += n_wg) {
+    int64_t x0 = i;
+    const int64_t rec = split_off(x0, a.hkv);
+    const int g = (int)x0;
+    const int4 c = uniform4(a.comb_seqs + rec);
+    const int splits = c.z & 0xffffff, rows = (c.z >> 24) + 1;
+    if ((unsigned)c.x >= (unsigned)a.batch || c.y < 0 || splits < 1 || rows > kCombRows || c.w < 0 ||
+        c.w + rows > a.total_q || (int64_t)c.y + (int64_t)rows * splits > a.slot_cap)
+      continue;
+    for (int t = hx::tid_x(); t < rows * per_row; t += kWideThreads) {
+      const int r = t / per_row, rem = t - r * per_row, h = rem / quads, d0 = 4 * (rem - h * quads);
+      const int qh = g * ws.group + h;
+      const int64_t base = ((int64_t)c.y + (int64_t)r * splits) * a.hq + qh;
+      float m = -INFINITY, l = 0.f, x[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int s0 = 0; s0 < splits; s0 += 4) {  // four splits' loads together
+        float2 ml[4];
+        float4 o4[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int64_t at = base + (int64_t)min(s0 + j, splits - 1) * a.hq;
+          ml[j] = a.part_ml[at];
+          o4[j] = *reinterpret_cast<const float4*>(part_o + at * D + d0);
+        }
+        float mn = m;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mn = fmaxf(mn, ml[j].x);
+        if (mn == -INFINITY) continue;
+        const float alpha = m == -INFINITY ? 0.f : hx::fast_exp2(m - mn);
+        l *= alpha;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] *= alpha;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const bool live = s0 + j < splits && ml[j].x != -INFINITY;
+          const float wt = live ? hx::fast_exp2(ml[j].x - mn) : 0.f;
+          l = fmaf(wt, ml[j].y, l);
+          x[0] = fmaf(wt, o4[j].x, x[0]);
+          x[1] = fmaf(wt, o4[j].y, x[1]);
+          x[2] = fmaf(wt, o4[j].z, x[2]);
+          x[3] = fmaf(wt, o4[j].w, x[3]);
+        }
+        m = mn;
+      }
+      const float inv = l > 0.f ? 1.f / l : 0.f;
+      const int64_t orow = c.w + r;
+      *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + orow * a.o_row + (int64_t)qh * a.o_head + d0) =
+          make_uint2(hx::pack2_round<T>(x[0] * inv, x[1] * inv), hx::pack2_round<T>(x[2] * inv, x[3] * inv));
+      if (a.lse && d0 == 0)
+        a.lse[(int64_t)qh * a.total_q + orow] = l > 0.f ? (m + (log2f(l) - wide_p_shift<T>())) * kLn2 : -INFINITY;
+    }
   }
 }
 
@@ -2356,7 +2690,7 @@ int launch_run_g(const RunArgs& a, const RunArgs* side_pf, int G, hipStream_t s)
 }
 
 // head_dim 128 with G in {1, 2, 4, 8} runs the decode / chunk / combine kernels; every
-// other supported shape runs generic_kernel.
+// other supported shape runs wide_kernel.
 bool tuned_shape(int G, int head_dim) { return head_dim == kD && valid_group(G); }
 
 int check_shape(int batch, int max_q, int max_k, int hq, int hkv, int head_dim) {
@@ -2366,20 +2700,36 @@ int check_shape(int batch, int max_q, int max_k, int hq, int hkv, int head_dim) 
   return HX_OK;
 }
 
+// The layout of a plan for wide_kernel, and whether it holds work lists: the lists and
+// fp32 partials when the workspace has room for them, else sequence info alone (every
+// block whole). The plan's stamp names the choice. make_layout's size is enough for any
+// shape.
+Layout wide_layout(int batch, int max_q, int max_k, int hq, int hkv, int head_dim) {
+  return make_layout(batch, max_q, max_k, hq, hkv, wide_geometry(hq, hkv), head_dim * sizeof(float));
+}
+Layout pick_wide_layout(int batch, int max_q, int max_k, int hq, int hkv, int head_dim, size_t bytes, bool* lists) {
+  const Layout l = wide_layout(batch, max_q, max_k, hq, hkv, head_dim);
+  *lists = l.total <= bytes;
+  return *lists ? l : wide_plain_layout(batch);
+}
+
 template <typename T>
-int launch_generic(const RunArgs& a, const GenericShape& gs, hipStream_t s) {
-  const int64_t grid = (int64_t)a.batch * gs.row_blocks * a.hkv * gs.head_blocks;
-  if (grid > INT32_MAX) return HX_E_INVALID_ARG;
-  if (grid == 0) return HX_OK;
-  const dim3 g3((unsigned)grid), b3(256);
-  if (gs.head_dim <= 32)
-    hipLaunchKernelGGL((generic_kernel<T, 32>), g3, b3, 0, s, a, gs);
-  else if (gs.head_dim <= 64)
-    hipLaunchKernelGGL((generic_kernel<T, 64>), g3, b3, 0, s, a, gs);
-  else if (gs.head_dim <= 128)
-    hipLaunchKernelGGL((generic_kernel<T, 128>), g3, b3, 0, s, a, gs);
-  else
-    hipLaunchKernelGGL((generic_kernel<T, 256>), g3, b3, 0, s, a, gs);
+int launch_wide(const RunArgs& a, const WideShape& ws, hipStream_t s) {
+  const int64_t work = ws.lists ? (ws.max_pf + a.dec_cap * ws.dec_head_blocks) * a.hkv
+                                : (int64_t)a.batch * ws.row_blocks * ws.head_blocks * a.hkv;
+  if (work == 0) return HX_OK;
+  const int wgs = (int)(work < kWideWGs ? work : kWideWGs);
+  const dim3 grid((unsigned)wgs), block(kWideThreads);
+  if (ws.head_dim <= 32) hipLaunchKernelGGL((wide_kernel<T, 32>), grid, block, 0, s, a, ws, wgs);
+  else if (ws.head_dim <= 64) hipLaunchKernelGGL((wide_kernel<T, 64>), grid, block, 0, s, a, ws, wgs);
+  else if (ws.head_dim <= 96) hipLaunchKernelGGL((wide_kernel<T, 96>), grid, block, 0, s, a, ws, wgs);
+  else if (ws.head_dim <= 128) hipLaunchKernelGGL((wide_kernel<T, 128>), grid, block, 0, s, a, ws, wgs);
+  else hipLaunchKernelGGL((wide_kernel<T, 256>), grid, block, 0, s, a, ws, wgs);
+  if (ws.lists && ws.max_comb > 0) {
+    const int64_t merges = ws.max_comb * a.hkv;
+    const int cw = (int)(merges < kWideWGs ? merges : kWideWGs);
+    hipLaunchKernelGGL((wide_combine_kernel<T>), dim3((unsigned)cw), block, 0, s, a, ws, cw);
+  }
   return hx::status_from_hip(hipGetLastError());
 }
 
@@ -2390,7 +2740,10 @@ extern "C" {
 size_t hx_varlen_attn_workspace_bytes(int32_t batch, int32_t max_q, int32_t max_k,
                                       int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim) {
   if (check_shape(batch, max_q, max_k, n_q_heads, n_kv_heads, head_dim) != HX_OK) return 0;
-  return make_layout(batch, max_q, max_k, n_q_heads, n_kv_heads).total;
+  const size_t least = make_layout(batch, max_q, max_k, n_q_heads, n_kv_heads).total;
+  if (tuned_shape(n_q_heads / n_kv_heads, head_dim)) return least;
+  const size_t wide = wide_layout(batch, max_q, max_k, n_q_heads, n_kv_heads, head_dim).total;
+  return wide > least ? wide : least;
 }
 
 size_t hx_varlen_attn_error_word_offset(void) { return H_ERR * sizeof(int32_t); }
@@ -2474,11 +2827,20 @@ int hx_varlen_attn_plan(const int32_t* cu_seq_q, const int32_t* cu_seq_k,
   if (page_size == 0 && (!cu_seq_k || total_k_rows < 0)) return HX_E_INVALID_ARG;
   if (batch > 0 && !cu_seq_q) return HX_E_INVALID_ARG;
   if (batch > 0 && !seqused_k && !cu_seq_k) return HX_E_INVALID_ARG;
-  const Layout l = make_layout(batch, max_q, max_k, n_q_heads, n_kv_heads);
+  Layout l = make_layout(batch, max_q, max_k, n_q_heads, n_kv_heads);
   if (!workspace || (uintptr_t)workspace % 256 || workspace_bytes < l.total) return HX_E_WORKSPACE;
   uint8_t* ws = static_cast<uint8_t*>(workspace);
-  const Geometry geo = geometry(n_q_heads, n_kv_heads);
+  Geometry geo = geometry(n_q_heads, n_kv_heads);
   PlanArgs a;
+  a.stamp = kPlanStamp;
+  a.plain = 0;
+  if (!tuned_shape(geo.G, head_dim)) {
+    bool lists;
+    l = pick_wide_layout(batch, max_q, max_k, n_q_heads, n_kv_heads, head_dim, workspace_bytes, &lists);
+    geo = wide_geometry(n_q_heads, n_kv_heads);
+    a.stamp = wide_stamp(head_dim) + (lists ? 1 : 0);
+    a.plain = !lists;
+  }
   a.cu_q = cu_seq_q;
   a.cu_k = cu_seq_k;
   a.used_k = seqused_k;
@@ -2582,9 +2944,13 @@ int run_impl(const void* q, int64_t q_row_stride, int64_t q_head_stride,
     return HX_E_INVALID_ARG;
   // Per-split row offsets are 32-bit: 256 rows of kv_row_stride must fit.
   if (kv_row_stride > (int64_t)(1 << 23)) return HX_E_INVALID_ARG;
-  const Layout l = make_layout(batch, max_q, max_k, n_q_heads, n_kv_heads);
+  Layout l = make_layout(batch, max_q, max_k, n_q_heads, n_kv_heads);
   if (!workspace || (uintptr_t)workspace % 256 || workspace_bytes < l.total) return HX_E_WORKSPACE;
   if (batch == 0) return HX_OK;
+  const bool tuned = tuned_shape(n_q_heads / n_kv_heads, head_dim);
+  bool wide_lists = false;
+  if (!tuned)
+    l = pick_wide_layout(batch, max_q, max_k, n_q_heads, n_kv_heads, head_dim, workspace_bytes, &wide_lists);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   RunArgs a;
   a.q = static_cast<const uint8_t*>(q);
@@ -2760,7 +3126,6 @@ int run_impl(const void* q, int64_t q_row_stride, int64_t q_head_stride,
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int G = n_q_heads / n_kv_heads;
-  const bool tuned = tuned_shape(G, head_dim);
   if (app != nullptr && total_q > 0) {
     if (!app->k_new || !app->v_new || !app->write_slots) return HX_E_INVALID_ARG;
     // Write slots index pool rows of n_kv_heads * head_dim contiguous elements (the pool
@@ -2772,11 +3137,11 @@ int run_impl(const void* q, int64_t q_row_stride, int64_t q_head_stride,
         app->kn_head % 8 || app->vn_row % 8 || app->vn_head % 8 || app->kn_row < 0 ||
         app->kn_head < 0 || app->vn_row < 0 || app->vn_head < 0 || app->pool_rows < 0)
       return HX_E_INVALID_ARG;
-    // Chunk rows (and every row of generic_kernel) read their own new keys from the
+    // Chunk rows (and every row of wide_kernel) read their own new keys from the
     // pool. When the tick may hold chunk rows and a decode launch runs on the tuned path,
     // workgroups added to that launch write every row (the chunk kernel runs after it,
     // also in a later call); a decode-only tick's rows are written by their own decode
-    // workgroups; otherwise (chunk rows run, the generic kernel runs, or this call
+    // workgroups; otherwise (chunk rows run, wide_kernel runs, or this call
     // launches neither decode nor chunk work) every row is appended first, so that a
     // call given new rows always writes them.
     const bool append_in_decode = tuned && max_q >= 2 && a.grid_dec > 0;
@@ -2803,12 +3168,24 @@ int run_impl(const void* q, int64_t q_row_stride, int64_t q_head_stride,
     }
   }
   if (!tuned) {
-    // One kernel covers every row; a call whose hints launch neither decode nor chunk
-    // work (the combine-only phase of a split run) launches nothing.
+    // One launch covers every row, a second merges its splits; a call whose hints launch
+    // neither decode nor chunk work (the combine-only phase of a split run) launches nothing.
     if (decode_items_hint == 0 && prefill_items_hint == 0) return HX_OK;
-    const GenericShape gs = generic_shape(max_q, G, head_dim);
-    if (dtype == HX_DTYPE_BF16) return launch_generic<__bf16>(a, gs, s);
-    return launch_generic<_Float16>(a, gs, s);
+    const Geometry geo = wide_geometry(n_q_heads, n_kv_heads);
+    WideShape shape;
+    shape.head_dim = head_dim;
+    shape.group = G;
+    shape.heads = geo.Gw;
+    shape.rows = geo.rows_per_item;
+    shape.head_blocks = geo.head_quads;
+    shape.dec_head_blocks = (int32_t)ceil_div(G, kWideDecUnits);
+    shape.row_blocks = (int32_t)ceil_div(max_q > 0 ? max_q : 1, geo.rows_per_item);
+    shape.lists = wide_lists;
+    shape.stamp = wide_stamp(head_dim);
+    shape.max_pf = l.max_pf;
+    shape.max_comb = l.max_comb;
+    if (dtype == HX_DTYPE_BF16) return launch_wide<__bf16>(a, shape, s);
+    return launch_wide<_Float16>(a, shape, s);
   }
   const RunArgs* side = has_side_pf ? &side_pf : nullptr;
   if (dtype == HX_DTYPE_BF16) return launch_run_g<__bf16>(a, side, G, s);

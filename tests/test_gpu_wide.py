@@ -1,0 +1,95 @@
+"""The any-head_dim attention kernel at the edges of its splits: units per block (64 (row,
+head) pairs, 16 per decode item), 64-key tiles, 256-key decode splits, padded head dims,
+and the form without work lists, against the float64 oracle."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from helios_amd import ops, synth
+from tests.gpu_cases import DeviceTick, compare, say
+
+pytestmark = pytest.mark.gpu
+
+
+def _tick(q_lens, k_lens, hq, hkv, d, dtype, device, seed):
+    free = [int(x) for x in synth.permutation(seed, sum(-(-k // 256) for k in k_lens) + 2)]
+    tables = synth._assign_pages(k_lens, free, 256)
+    w = synth.Workload(f"wide{seed}", list(q_lens), [k - n for n, k in zip(q_lens, k_lens)], tables, len(free),
+                       n_q_heads=hq, n_kv_heads=hkv, head_dim=d, seed=seed)
+    return DeviceTick(w, dtype, device)
+
+
+# One-token rows around the tile and split edges, then chunks around the unit-block edges.
+Q_LENS = [1, 1, 1, 1, 1, 1, 1, 2, 3, 16, 17, 22, 65]
+K_LENS = [1, 64, 65, 256, 257, 513, 1090, 2, 70, 16, 300, 257, 641]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", [(3, 3, 8), (4, 2, 24), (8, 2, 64), (6, 2, 72), (17, 1, 96), (6, 1, 128),
+                                      (70, 1, 32), (32, 1, 136), (4, 1, 256)])
+def test_wide_edges(device, hq, hkv, d, dtype):
+    say("wide edges", hq, hkv, d, dtype)
+    tick = _tick(Q_LENS, K_LENS, hq, hkv, d, dtype, device, 300 + d)
+    for window in ((-1, 0), (100, 5)):
+        ref, ref_lse = tick.oracle(window=window)
+        out, lse = tick.attend(window=window, exact_grid=True, return_lse=True)
+        compare(out, ref, what=f"wide {hq}/{hkv} d={d} {window}")
+        # fp32 sums of at most 1090 terms, against float64
+        assert np.abs(lse.cpu().numpy() - ref_lse).max() < 1e-4
+
+
+def test_wide_keeps_p_in_more_than_16_bits(device):
+    """With V near 1 every output is a sum of many p times nearly the same value: rounding p
+    to bf16 before the product, with l summed unrounded, would show as 2^-9 of the output
+    with random sign; the output's own rounding is bounded by half its spacing."""
+    tick = _tick([1, 40], [1500, 700], 8, 2, 64, torch.bfloat16, device, 41)
+    tick.v_pool.fill_(1.0)
+    tick.v_pool[..., ::2] = 0.75
+    out = tick.attend()
+    torch.cuda.synchronize()
+    # exact weights of one sum to 1: both values are representable, so the result rounds to them
+    assert (out[..., 1::2] == 1.0).all() and (out[..., ::2] == 0.75).all()
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(4, 1, 256), (8, 1, 136)])
+def test_wide_without_work_lists(device, hq, hkv, d, monkeypatch):
+    """A workspace of the 16-bit partials' size (the least accepted) holds no fp32 partials at
+    these head dims and chunks of a few rows: the same results from whole rows."""
+    say("wide plain", hq, hkv, d)
+    tick = _tick([min(n, 3) for n in Q_LENS], K_LENS, hq, hkv, d, torch.bfloat16, device, 500 + d)
+    ref, ref_lse = tick.oracle()
+    sized = ops.workspace_bytes
+    least = sized(tick.w.batch, tick.w.max_q, tick.w.max_k, hq, hkv, 128)
+    assert least < sized(tick.w.batch, tick.w.max_q, tick.w.max_k, hq, hkv, d)
+    monkeypatch.setattr(ops, "workspace_bytes", lambda *a: least)
+    out, lse = tick.attend(exact_grid=True, return_lse=True)
+    compare(out, ref, what=f"wide plain {hq}/{hkv} d={d}")
+    assert np.abs(lse.cpu().numpy() - ref_lse).max() < 1e-4
+    # a plan with lists, run with the smaller size: whole rows again
+    monkeypatch.setattr(ops, "workspace_bytes", sized)
+    plan = tick.plan()
+    plan.ws_bytes = least
+    again = plan.run(tick.q, tick.k_pool, tick.v_pool, tick.block_table)
+    assert plan.error_word() == 0 and torch.equal(again.view(torch.int16), out.view(torch.int16))
+    monkeypatch.setattr(ops, "workspace_bytes", lambda *a: least - 256)
+    with pytest.raises(ValueError):
+        tick.plan()
+
+
+def test_wide_expanded_packed_keys(device):
+    """Packed keys whose row stride is 0 (one key broadcast over the sequence)."""
+    say("wide stride 0")
+    g = torch.Generator(device=device).manual_seed(3)
+    q = torch.randn(5, 6, 64, generator=g, device=device).to(torch.bfloat16)
+    k = torch.randn(1, 2, 64, generator=g, device=device).to(torch.bfloat16).expand(90, 2, 64)
+    v = torch.randn(1, 2, 64, generator=g, device=device).to(torch.bfloat16).expand(90, 2, 64)
+    cu_q = torch.tensor([0, 1, 5], dtype=torch.int32, device=device)
+    cu_k = torch.tensor([0, 20, 90], dtype=torch.int32, device=device)
+    out = ops.varlen_attn(q, k, v, cu_q, cu_k, 4, 70, is_causal=True, enable_gqa=True)
+    torch.cuda.synchronize()
+    want = v[0].repeat_interleave(3, dim=0).expand(5, 6, 64)
+    # equal weights of one row: the row itself, up to the rounding of fp32 sums
+    assert torch.equal(out, want)
