@@ -583,7 +583,8 @@ constexpr int kPlanChunkSeqs = 1024;
 constexpr int kPlanBlocks = 4096;
 constexpr int kPlanSearchWork = 1 << 16;  // candidates x blocks evaluated in one pass
 constexpr int kPlanSortBlocks = 256;
-static_assert(2 * kPlanSortBlocks <= kPlanThreads, "sort keys and item counts share the search buffer");
+static_assert(3 * kPlanSortBlocks <= kPlanThreads, "sort keys, item counts and ranks share the search buffer");
+static_assert(4 * kPlanSortBlocks <= kPlanThreads, "at least four threads rank each block");
 
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   __shared__ int wave_tot[kPlanThreads / 64];
@@ -703,12 +704,17 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   if (st0 > 0 && tm.y > st0) {
     const int ncand = tm.y - st0;  // candidates st0 + 1 .. max tiles
     if (ncand < kPlanThreads && (int64_t)(ncand + 1) * n_blk <= kPlanSearchWork) {
-      // Thread j <= ncand counts the workgroups at split size st0 + j; the smallest
-      // fitting candidate wins an LDS atomicMin.
-      if (tid <= ncand) {
+      // Workgroups at split size st0 + j for every j <= ncand, the blocks dealt over as many
+      // threads as there are per candidate (one thread walking all blocks took 0.08 us a
+      // block); the smallest fitting candidate wins an LDS atomicMin.
+      const int parts = kPlanThreads / (ncand + 1);
+      const int part = tid / (ncand + 1), j = tid - part * (ncand + 1);
+      if (tid <= ncand) cand_wgs[tid] = 0;
+      __syncthreads();
+      if (part < parts && part < n_blk) {
         int wg = 0;
-        for (int i = 0; i < n_blk; ++i) wg += chunk_split_count(fb_tiles[i], st0 + tid);
-        cand_wgs[tid] = wg;
+        for (int i = part; i < n_blk; i += parts) wg += chunk_split_count(fb_tiles[i], st0 + j);
+        atomicAdd(&cand_wgs[j], wg);
       }
       __syncthreads();
       const int64_t w0 = (int64_t)cand_wgs[0] * a.head_quads * a.hkv;
@@ -833,12 +839,28 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   const bool by_length = n_blk > 0 && n_blk <= kPlanSortBlocks;
   int* const blk_key = cand_wgs;                      // free after the split search
   int* const blk_items = cand_wgs + kPlanSortBlocks;
+  int* const blk_first = cand_wgs + 2 * kPlanSortBlocks;  // first item of the block
   if (by_length) {
     if (tid < n_blk) {
       const int S = chunk_split_count(fb_tiles[tid], split_tiles, keep_tiles);
       blk_key[tid] = (fb_tiles[tid] + S - 1) / S;
       blk_items[tid] = S * a.head_quads;
     }
+    __syncthreads();
+    // 16 threads rank each block (4 when there are more than 64 blocks): items of the
+    // blocks that go before it.
+    const int sh = n_blk <= kPlanThreads / 16 ? 4 : 2;
+    const int i = tid >> sh;
+    int before = 0;
+    if (i < n_blk) {
+      const int key = blk_key[i];
+      for (int j = tid & ((1 << sh) - 1); j < n_blk; j += 1 << sh) {
+        const int kj = blk_key[j];
+        before += kj > key || (kj == key && j < i) ? blk_items[j] : 0;
+      }
+    }
+    for (int m = 1; m < (1 << sh); m <<= 1) before += __shfl_xor(before, m);
+    if (i < n_blk && (tid & ((1 << sh) - 1)) == 0) blk_first[i] = before;
     __syncthreads();
   }
   for (int i = tid; i < n_blk; i += kPlanThreads) {
@@ -850,14 +872,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
     const int S = chunk_split_count(fb_tiles[i], split_tiles, keep_tiles);
     const int rows = min(a.rows_per_item, n - row0);
     int item0 = cs_off_p[k] + fb_p[i] - fb_p[f0];
-    if (by_length) {
-      const int key = blk_key[i];
-      item0 = 0;
-      for (int j = 0; j < n_blk; ++j) {
-        const int kj = blk_key[j];
-        item0 += kj > key || (kj == key && j < i) ? blk_items[j] : 0;
-      }
-    }
+    if (by_length) item0 = blk_first[i];
     const int slot = cs_off_s[k] + fb_s[i] - fb_s[f0];
     const int comb0 = cs_off_c[k] + fb_c[i] - fb_c[f0];
     const bool fits = S == 1 || slot + rows * S <= a.cslot_cap;
