@@ -18,7 +18,8 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC = PACKAGE_DIR / "csrc"
 INCLUDE = PACKAGE_DIR.parent / "include"
 LIBRARY = PACKAGE_DIR / "libhelios_paged.so"
-SOURCES = ("kv_ops.hip", "paged_attn.hip", "tick_meta.hip", "qk_rope.hip", "block_ops.hip", "logits.hip")
+SOURCES = ("kv_ops.hip", "paged_attn.hip", "tick_meta.hip", "qk_rope.hip", "block_ops.hip", "skinny_gemm.hip",
+           "logits.hip")
 ARCH = "gfx950"
 
 

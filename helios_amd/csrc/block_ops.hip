@@ -19,13 +19,6 @@ namespace {
 
 constexpr int kBlThreads = 256;
 
-// a + b, each an element pair, rounded like the element type's add.
-template <typename T>
-__device__ __forceinline__ uint32_t add2(uint32_t a, uint32_t b) {
-  return hx::pack2_round<T>(__fadd_rn(hx::Elem<T>::lo(a), hx::Elem<T>::lo(b)),
-                            __fadd_rn(hx::Elem<T>::hi(a), hx::Elem<T>::hi(b)));
-}
-
 __device__ __forceinline__ float row_rsqrt(float ss, int hidden, float eps, float* s_part) {
   ss = hx::wave_sum_xor(ss, 1, 32);
   if ((hx::tid_x() & 63) == 0) s_part[hx::tid_x() >> 6] = ss;
@@ -75,8 +68,8 @@ __global__ __launch_bounds__(kBlThreads) void add_rms_norm_vec_kernel(NormArgs a
     const int v = tid + i * kBlThreads;
     if (v >= nv) continue;
     if (a.y != nullptr) {
-      u[i] = make_uint4(add2<T>(u[i].x, yv[i].x), add2<T>(u[i].y, yv[i].y), add2<T>(u[i].z, yv[i].z),
-                        add2<T>(u[i].w, yv[i].w));
+      u[i] = make_uint4(hx::add2<T>(u[i].x, yv[i].x), hx::add2<T>(u[i].y, yv[i].y),
+                        hx::add2<T>(u[i].z, yv[i].z), hx::add2<T>(u[i].w, yv[i].w));
       reinterpret_cast<uint4*>(a.sum + row * a.hidden)[v] = u[i];
     }
     const uint32_t wd[4] = {u[i].x, u[i].y, u[i].z, u[i].w};
@@ -112,7 +105,7 @@ __global__ __launch_bounds__(kBlThreads) void add_rms_norm_kernel(NormArgs a) {
   const uint16_t* x = a.x + row * a.x_row;
   auto element = [&](int e) {
     uint32_t b = x[e];
-    if (a.y != nullptr) b = add2<T>(b, a.y[row * a.y_row + e]) & 0xffffu;
+    if (a.y != nullptr) b = hx::add2<T>(b, a.y[row * a.y_row + e]) & 0xffffu;
     return b;
   };
   float ss = 0.f;
@@ -126,14 +119,6 @@ __global__ __launch_bounds__(kBlThreads) void add_rms_norm_kernel(NormArgs a) {
   for (int e = tid; e < a.hidden; e += kBlThreads)
     a.norm[row * a.hidden + e] =
         hx::Elem<T>::bits(__fmul_rn(__fmul_rn(hx::Elem<T>::lo(element(e)), r), a.w[e]));
-}
-
-// silu(g) * u on an element pair: x / (1 + e^-x) in fp32, rounded, times u, rounded.
-template <typename T>
-__device__ __forceinline__ uint32_t swiglu2(uint32_t g, uint32_t u) {
-  const uint32_t s = hx::pack2_round<T>(hx::silu(hx::Elem<T>::lo(g)), hx::silu(hx::Elem<T>::hi(g)));
-  return hx::pack2_round<T>(__fmul_rn(hx::Elem<T>::lo(s), hx::Elem<T>::lo(u)),
-                            __fmul_rn(hx::Elem<T>::hi(s), hx::Elem<T>::hi(u)));
 }
 
 struct SwigluArgs {
@@ -150,8 +135,8 @@ __global__ __launch_bounds__(kBlThreads) void swiglu_vec_kernel(SwigluArgs a) {
   const int64_t r = i / a.ffn, c = i - r * a.ffn;
   const uint4* p = reinterpret_cast<const uint4*>(a.gate_up + r * a.row) + c;
   const uint4 g = p[0], u = p[a.ffn];
-  reinterpret_cast<uint4*>(a.out)[i] = make_uint4(swiglu2<T>(g.x, u.x), swiglu2<T>(g.y, u.y), swiglu2<T>(g.z, u.z),
-                                                  swiglu2<T>(g.w, u.w));
+  reinterpret_cast<uint4*>(a.out)[i] = make_uint4(hx::swiglu2<T>(g.x, u.x), hx::swiglu2<T>(g.y, u.y),
+                                                  hx::swiglu2<T>(g.z, u.z), hx::swiglu2<T>(g.w, u.w));
 }
 
 template <typename T>
@@ -160,7 +145,7 @@ __global__ __launch_bounds__(kBlThreads) void swiglu_kernel(SwigluArgs a) {
   if (i >= a.total) return;
   const int64_t r = i / a.ffn, c = i - r * a.ffn;
   const uint16_t* p = a.gate_up + r * a.row + c;
-  a.out[i] = (uint16_t)swiglu2<T>(p[0], p[a.ffn]);
+  a.out[i] = (uint16_t)hx::swiglu2<T>(p[0], p[a.ffn]);
 }
 
 template <typename T>

@@ -104,6 +104,21 @@ __device__ __forceinline__ uint32_t pack2_round<_Float16>(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){lo, hi}, h2));
 }
 
+// a + b, each an element pair, rounded like the element type's add.
+template <typename T>
+__device__ __forceinline__ uint32_t add2(uint32_t a, uint32_t b) {
+  return pack2_round<T>(__fadd_rn(Elem<T>::lo(a), Elem<T>::lo(b)),
+                            __fadd_rn(Elem<T>::hi(a), Elem<T>::hi(b)));
+}
+
+// silu(g) * u on an element pair: x / (1 + e^-x) in fp32, rounded, times u, rounded.
+template <typename T>
+__device__ __forceinline__ uint32_t swiglu2(uint32_t g, uint32_t u) {
+  const uint32_t s = pack2_round<T>(silu(Elem<T>::lo(g)), silu(Elem<T>::hi(g)));
+  return pack2_round<T>(__fmul_rn(Elem<T>::lo(s), Elem<T>::lo(u)),
+                            __fmul_rn(Elem<T>::hi(s), Elem<T>::hi(u)));
+}
+
 // Eight packed 1.0 values of element type T.
 template <typename T>
 __device__ __forceinline__ uint4 ones8();

@@ -4,8 +4,9 @@ Mirrors Qwen3Model._forward_packed (src/helios/runtime/qwen3/model.py:92-110) an
 TransformerBlock / GroupedQueryAttention / FeedForward forwards it runs
 (layers.py:13-27, :131-164, :202-232), with random-init weights (no checkpoint is
 fetched). This is the caller of the hot path, kept to measure it in place: torch runs
-the products on hipBLASLt, the steps between them are one launch each
-(``ops.add_rms_norm``, ``ops.swiglu``), and the attention step goes through
+the products on hipBLASLt, with one launch for each step between them
+(``ops.add_rms_norm``, ``ops.swiglu``), or, for a few rows, products that take those steps
+along (``ops.block_linear``), and the attention step goes through
 ``PackedBatchCache.attend_projected`` (fused q/k norm + RoPE + KV append, then paged
 attention). With ``fused_rope=False`` everything but the attention is the reference's own
 sequence of torch operations (norms, RoPE, SiLU, then ``attend``).
@@ -46,6 +47,12 @@ def _apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positions
     return (x * c + torch.cat((-x[..., half:], x[..., :half]), dim=-1) * s).to(x.dtype)
 
 
+# Ticks of at most this many rows run their products through ops.block_linear: a layer's four
+# products and the steps between them take 62-71 us that way and 102 us on hipBLASLt at up to
+# 16 rows (one MFMA row tile); at 17-32 rows hipBLASLt's take 77-82 us, a second row tile 88-94.
+FEW_ROWS = 16
+
+
 class PagedQwen3Decoder:
     """Random-init Qwen3 weights in the reference's layout, on one device."""
 
@@ -75,6 +82,14 @@ class PagedQwen3Decoder:
         self.final_norm = torch.ones(config.hidden_size, device=self.device)
         self.cos, self.sin = _rope_tables(config, self.device)
 
+    @staticmethod
+    def _few_rows(tokens: int, dtype: torch.dtype, layer: dict[str, torch.Tensor]) -> bool:
+        """Whether this layer's products go to ``ops.block_linear``: few rows, and weights it
+        can read."""
+        return tokens <= FEW_ROWS and dtype in (torch.bfloat16, torch.float16) and all(
+            w.is_contiguous() and w.dtype == dtype and w.data_ptr() % 16 == 0 and w.shape[0] % 32 == 0
+            and w.shape[1] % 64 == 0 for w in (layer["qkv"], layer["o"], layer["gate_up"], layer["down"]))
+
     @torch.inference_mode()
     def forward_packed(self, input_ids: torch.Tensor, cache: PackedBatchCache, *,
                        fused_rope: bool = True, attention_events: list | None = None,
@@ -95,11 +110,16 @@ class PagedQwen3Decoder:
         tokens = x.shape[1]
         branch = None  # the last branch's output, not yet added to the residual stream
         for index, layer in enumerate(self.layers):
-            if fused_rope:
+            few = fused_rope and self._few_rows(tokens, x.dtype, layer)
+            if few:
+                if branch is not None:
+                    x, branch = x + branch, None
+                qkv = ops.block_linear(x, layer["qkv"], norm_weight=layer["input_norm"], eps=eps)
+            elif fused_rope:
                 x, h = ops.add_rms_norm(x, branch, layer["input_norm"], eps)
+                qkv = h @ layer["qkv"].t()
             else:
-                h = _rms_norm(x, layer["input_norm"], eps)
-            qkv = h @ layer["qkv"].t()
+                qkv = _rms_norm(x, layer["input_norm"], eps) @ layer["qkv"].t()
             q, k, v = qkv[..., :hq], qkv[..., hq:hq + hkv], qkv[..., hq + hkv:]
             if attention_events is not None:
                 start = torch.cuda.Event(enable_timing=True)
@@ -119,6 +139,11 @@ class PagedQwen3Decoder:
                 end.record()
                 attention_events.append((start, end))
             context = context.transpose(1, 2).reshape(1, tokens, -1)
+            if few:
+                x = ops.block_linear(context, layer["o"], residual=x)
+                h = ops.block_linear(x, layer["gate_up"], norm_weight=layer["post_norm"], eps=eps, swiglu=True)
+                x = ops.block_linear(h, layer["down"], residual=x)
+                continue
             branch = context @ layer["o"].t()
             if fused_rope:
                 x, h = ops.add_rms_norm(x, branch, layer["post_norm"], eps)

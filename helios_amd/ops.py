@@ -328,6 +328,48 @@ def swiglu(gate_up: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def block_linear(x: torch.Tensor, weight: torch.Tensor, *, norm_weight: torch.Tensor | None = None,
+                 eps: float = 0.0, residual: torch.Tensor | None = None, swiglu: bool = False) -> torch.Tensor:
+    """``x @ weight.t()`` for ticks of up to 16 rows, with the decoder block's steps around it
+    (layers.py:13-40, :202-232) in the same launch: ``x`` RMSNormed first with
+    ``norm_weight``; ``residual`` added to the rounded product; ``swiglu``: ``weight`` holds
+    gate, then up rows, and the result is ``silu(gate) * up``. Values round to the dtype where
+    the separate steps round them. ``x`` ``[..., K]`` and ``residual`` ``[..., N]`` contiguous,
+    ``weight`` ``[N, K]`` (``[2 N, K]``) contiguous, bfloat16 or float16, K a multiple of 64
+    and N of 16."""
+    device = x.device
+    if device.type != "cuda" or weight.device != device:
+        _require_gpu(x, weight)
+    dtype = _SUPPORTED.get(x.dtype)
+    if dtype is None or weight.dtype != x.dtype:
+        raise ValueError("block_linear supports bfloat16 and float16 x and weight of one dtype.")
+    k = x.shape[-1]
+    if weight.ndim != 2 or weight.shape[1] != k or not weight.is_contiguous() or not x.is_contiguous():
+        raise ValueError("x must be contiguous [..., K] and weight contiguous [N, K].")
+    cols = weight.shape[0]
+    if swiglu:
+        if cols % 2 or residual is not None:
+            raise ValueError("swiglu takes a weight of gate and up rows and no residual.")
+        cols //= 2
+    shape = (*x.shape[:-1], cols)
+    if residual is not None and (residual.shape != shape or residual.dtype != x.dtype or residual.device != device
+                                 or not residual.is_contiguous()):
+        raise ValueError("residual must be contiguous, of the result's shape and dtype.")
+    if norm_weight is not None:
+        if tuple(norm_weight.shape) != (k,) or norm_weight.device != device or not norm_weight.is_floating_point():
+            raise ValueError("norm_weight must be floating-point [K].")
+        norm_weight = norm_weight.float().contiguous()  # no copy for the usual float32 vector
+    out = torch.empty(shape, dtype=x.dtype, device=device)
+    if k:
+        code = _capi.lib().hx_skinny_gemm(
+            x.data_ptr(), k, x.numel() // k, weight.data_ptr(), k, cols, k, dtype,
+            None if norm_weight is None else norm_weight.data_ptr(), eps,
+            None if residual is None else residual.data_ptr(), cols, 1 if swiglu else 0,
+            out.data_ptr(), cols, _stream_ptr(device))
+        _capi.check(code, "hx_skinny_gemm")
+    return out
+
+
 # --------------------------------------------------------------- logits and argmax
 class GreedyHeads(NamedTuple):
     """Result of ``final_norm_logits_argmax``: ``token_ids`` int64 ``[n]`` (-1 for an index

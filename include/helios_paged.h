@@ -510,6 +510,21 @@ int hx_add_rms_norm(const void* x, int64_t x_row_stride, const void* y, int64_t 
 int hx_swiglu(const void* gate_up, int64_t row_stride, int64_t rows, int32_t ffn,
               int32_t dtype, void* out, void* stream);
 
+/* The block's products for up to 16 rows (layers.py:13-27, :131-164), the steps above
+ * fused in: y = h weight^T with h = x, or its RMSNorm when norm_weight is given; out =
+ * round(y); residual + round(y) when residual is given; silu(round(y[:, :cols])) *
+ * round(y[:, cols:]) with swiglu (weight then holds 2 * cols rows, gate first; not
+ * together with residual). fp32 accumulation. x rows k elements, weight rows k elements,
+ * out and residual rows cols; strides in elements. HX_E_UNSUPPORTED for more than 16 rows,
+ * cols not a multiple of 16 or k not a multiple of 64; x, weight and norm_weight 16-byte
+ * aligned with row strides in multiples of 8, out and residual 4-byte aligned with even
+ * row strides (HX_E_INVALID_ARG otherwise). out must not overlap x or weight. */
+int hx_skinny_gemm(const void* x, int64_t x_row_stride, int64_t rows, const void* weight,
+                   int64_t weight_row_stride, int32_t cols, int32_t k, int32_t dtype,
+                   const float* norm_weight, float eps, const void* residual,
+                   int64_t residual_row_stride, int32_t swiglu, void* out,
+                   int64_t out_row_stride, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

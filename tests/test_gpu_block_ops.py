@@ -77,3 +77,51 @@ def test_add_rms_norm_and_swiglu_refuse_what_they_cannot_read(device):
         ops.add_rms_norm(x.float(), None, w, 1e-6)
     with pytest.raises(ValueError):
         ops.swiglu(x[:, :15])
+
+
+def _parts(x, w, norm, eps, residual, swiglu):
+    """The separate steps, rounding where they round."""
+    h = x if norm is None else _rms(x, norm, eps)
+    y = (h.double() @ w.double().t()).to(x.dtype)
+    if swiglu:
+        gate, up = y.chunk(2, dim=-1)
+        return torch.nn.functional.silu(gate) * up
+    return y if residual is None else residual + y
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols,k", [(1, 16, 64), (8, 48, 192), (9, 2560, 2560), (16, 32, 704), (15, 16, 9728)])
+def test_block_linear(device, rows, cols, k, dtype):
+    """Row counts around the half tiles, K slices that are empty, uneven and long, beyond
+    the part of a row that the norm's statistics hold in registers."""
+    say("block_linear", rows, cols, k, dtype)
+    g = torch.Generator(device=device).manual_seed(rows + cols + k)
+    x = torch.randn(1, rows, k, generator=g, device=device).to(dtype)
+    w = (torch.randn(2 * cols, k, generator=g, device=device) * k ** -0.5).to(dtype)
+    norm = 1 + 0.1 * torch.randn(k, generator=g, device=device)
+    residual = torch.randn(1, rows, cols, generator=g, device=device).to(dtype)
+    for n in (None, norm):
+        for kw in (dict(), dict(residual=residual), dict(swiglu=True)):
+            wt = w if kw.get("swiglu") else w[:cols]
+            got = ops.block_linear(x, wt, norm_weight=n, eps=1e-6, **kw).float()
+            ref = _parts(x, wt, n, 1e-6, kw.get("residual"), kw.get("swiglu", False)).float()
+            # fp32 sums of products of size 1/sqrt(k): y is right to k * 2^-24 of its terms'
+            # size, so its rounding may fall one step apart. A normalised x one step apart in
+            # one element moves y by ULP / sqrt(k) of one term, below that step. Through
+            # SwiGLU: one step of each factor and two roundings.
+            steps = 4 if kw.get("swiglu") else 2
+            size = 1 + ref.abs() + (residual.float().abs() if "residual" in kw else 0)
+            assert ((got - ref).abs() <= steps * ULP[dtype] * size).all(), (kw.keys(), n is None)
+            # and on average no further than the rounding of y itself
+            assert (got - ref).abs().mean() <= 0.1 * ULP[dtype]
+
+
+def test_block_linear_refuses_other_shapes(device):
+    x = torch.zeros(17, 64, dtype=torch.bfloat16, device=device)
+    w = torch.zeros(32, 64, dtype=torch.bfloat16, device=device)
+    for args in ((x, w), (x[:4], w[:8]), (x[:4, :32].contiguous(), w[:, :32].contiguous()), (x[:4], w[:, :32]),
+                 (x[:4].float(), w.float())):
+        with pytest.raises(ValueError):
+            ops.block_linear(*args)
+    with pytest.raises(ValueError):
+        ops.block_linear(x[:4], w, swiglu=True, residual=x[:4, :16].contiguous())
