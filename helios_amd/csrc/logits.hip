@@ -126,6 +126,32 @@ __device__ __forceinline__ void lg_load(uint4 (&rw)[8], uint4 (&rx)[NT], const u
   }
 }
 
+// Four logits of one row, vocab rows vr0 .. vr0 + 3: rounded to the model dtype, written out
+// when asked for, and their largest key.
+template <typename T>
+__device__ __forceinline__ uint64_t lg_finish(const hx::f32x4_t& acc, int64_t vr0, int64_t vocab, int tok, int n,
+                                              uint16_t* __restrict__ logits, int64_t ld_logits) {
+  uint16_t bits[4];
+  uint64_t best = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    bits[i] = hx::Elem<T>::bits(acc[i]);
+    const float f = hx::Elem<T>::lo((uint32_t)bits[i]);
+    if (vr0 + i < vocab) best = max_u64(best, argmax_key(f, (uint32_t)(vr0 + i)));
+  }
+  if (logits != nullptr && tok < n) {
+    uint16_t* dst = logits + (int64_t)tok * ld_logits + vr0;
+    if (vr0 + 3 < vocab && ((reinterpret_cast<uintptr_t>(dst) & 7) == 0)) {
+      *reinterpret_cast<uint2*>(dst) = make_uint2(hx::pack2(bits[0], bits[1]), hx::pack2(bits[2], bits[3]));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (vr0 + i < vocab) dst[i] = bits[i];
+    }
+  }
+  return best;
+}
+
 // ------------------------------------------------------------------- logits + argmax
 // Workgroup g owns vocab rows [128 g, 128 g + 128); wave w of it owns 32 of them as two
 // 16-row MFMA tiles, against all NT 16-row tiles of the normalised logit rows. The
@@ -202,23 +228,7 @@ __global__ __launch_bounds__(kLgThreads) void logits_argmax_kernel(
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
       const int64_t vr0 = v0 + 32 * wave + 16 * v + 4 * (lane >> 4);
-      uint16_t bits[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bits[i] = hx::Elem<T>::bits(acc[v][t][i]);
-        const float f = hx::Elem<T>::lo((uint32_t)bits[i]);
-        if (vr0 + i < vocab) best = max_u64(best, argmax_key(f, (uint32_t)(vr0 + i)));
-      }
-      if (logits != nullptr && tok < n) {
-        uint16_t* dst = logits + (int64_t)tok * ld_logits + vr0;
-        if (vr0 + 3 < vocab && ((reinterpret_cast<uintptr_t>(dst) & 7) == 0)) {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(hx::pack2(bits[0], bits[1]), hx::pack2(bits[2], bits[3]));
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (vr0 + i < vocab) dst[i] = bits[i];
-        }
-      }
+      best = max_u64(best, lg_finish<T>(acc[v][t], vr0, vocab, tok, n, logits, ld_logits));
     }
     best = max_u64(best, shfl_xor_u64(best, 16));
     best = max_u64(best, shfl_xor_u64(best, 32));
@@ -227,6 +237,137 @@ __global__ __launch_bounds__(kLgThreads) void logits_argmax_kernel(
   __syncthreads();
   for (int j = tid; j < n; j += kLgThreads) {
     const uint64_t m = max_u64(max_u64(s_key[0][j], s_key[1][j]), max_u64(s_key[2][j], s_key[3][j]));
+    partial[(int64_t)j * tiles + hx::wg_x()] = m;
+  }
+}
+
+// The same product for many logit rows, where reading fragments from LDS costs more than the
+// weight stream: 8 waves x 5 MFMA tiles of vocab rows, so that an x fragment read feeds five
+// MFMAs instead of two, in one workgroup per CU (HBM and MFMA bound in turn: 129 rows take
+// 177 us, 4.4 TB/s of weights and 0.63 PFLOP/s; 64 rows and fewer are faster above). Weights and x go from memory straight into
+// LDS, 32 hidden elements at a time, into three buffers used in turn: two chunks are in
+// flight while one is consumed, and a chunk costs one wait and one barrier.
+//
+// LDS rows are 64 bytes; the 16-byte piece at position p of row r is piece p ^ ((r >> 2) & 3),
+// so a fragment read's 16 rows hit 16 distinct 16-byte bank groups. A load instruction
+// fills 16 rows (lane l: row l >> 2, position l & 3); a wave loads its own weight rows.
+constexpr int kLtWaves = 8, kLtVT = 5;
+constexpr int kLtThreads = 64 * kLtWaves;
+constexpr int kLtVocab = 16 * kLtVT * kLtWaves;  // vocab rows per workgroup: 640
+constexpr int kLtTileBytes = 16 * 64;            // a 16-row tile of a chunk
+
+template <int NT>
+struct LtBuf {
+  unsigned char w[kLtWaves * kLtVT * kLtTileBytes];
+  unsigned char x[NT * kLtTileBytes];
+};
+
+template <typename T, int NT>
+__global__ __launch_bounds__(kLtThreads, 2) void logits_argmax_wide_kernel(
+    const uint16_t* __restrict__ emb, int64_t ld_emb, int64_t vocab, int hidden,
+    const uint16_t* __restrict__ xn, int n, int32_t tiles, uint64_t* __restrict__ partial,
+    uint16_t* __restrict__ logits, int64_t ld_logits) {
+  // Each buffer its own variable: a read of one does not wait for copies into another.
+  __shared__ __attribute__((aligned(16))) LtBuf<NT> buf0;
+  __shared__ __attribute__((aligned(16))) LtBuf<NT> buf1;
+  __shared__ __attribute__((aligned(16))) LtBuf<NT> buf2;
+  constexpr int XL = NT > kLtWaves ? 2 : 1;  // x loads per wave and chunk (spare ones repeat a tile)
+
+  const int tid = hx::tid_x(), lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t v0 = (int64_t)hx::wg_x() * kLtVocab;
+  const int rows = (int)min((int64_t)kLtVocab, vocab - v0);
+
+  const uint32_t ld_bytes = (uint32_t)ld_emb * 2u;
+  const __amdgpu_buffer_rsrc_t wres =
+      hx::buffer_rsrc(emb + v0 * ld_emb, (uint32_t)(rows - 1) * ld_bytes + (uint32_t)hidden * 2u);
+  const __amdgpu_buffer_rsrc_t xres = hx::buffer_rsrc(xn, (uint32_t)(NT * 16) * (uint32_t)hidden * 2u);
+  uint32_t woff[kLtVT], xoff[XL];
+  int xtile[XL];
+  const int lrow = lane >> 2, lpiece = (lane & 3) ^ ((lrow >> 2) & 3);
+#pragma unroll
+  for (int v = 0; v < kLtVT; ++v)  // rows past the vocab re-read the last row (never used)
+    woff[v] = (uint32_t)min(16 * (kLtVT * w + v) + lrow, rows - 1) * ld_bytes + 16u * (uint32_t)lpiece;
+#pragma unroll
+  for (int j = 0; j < XL; ++j) {
+    xtile[j] = min(w + j * kLtWaves, NT - 1);
+    xoff[j] = (uint32_t)(16 * xtile[j] + lrow) * (uint32_t)hidden * 2u + 16u * (uint32_t)lpiece;
+  }
+  auto load = [&](LtBuf<NT>& b, int c) __attribute__((always_inline)) {
+    const uint32_t k = 64u * (uint32_t)c;  // bytes
+#pragma unroll
+    for (int v = 0; v < kLtVT; ++v) hx::ld16_to_lds(wres, b.w + (kLtVT * w + v) * kLtTileBytes, woff[v] + k);
+#pragma unroll
+    for (int j = 0; j < XL; ++j) hx::ld16_to_lds(xres, b.x + xtile[j] * kLtTileBytes, xoff[j] + k);
+  };
+
+  hx::f32x4_t acc[kLtVT][NT];
+#pragma unroll
+  for (int v = 0; v < kLtVT; ++v)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[v][t] = hx::f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int chunks = hidden / 32;
+  const int frag = 64 * (lane & 15) + 16 * ((lane >> 4) ^ ((lane >> 2) & 3));  // row lane & 15, piece lane >> 4
+  auto step = [&](int c, const LtBuf<NT>& cur, LtBuf<NT>& next, bool steady) __attribute__((always_inline)) {
+    // Chunk c has landed for this wave (chunk c + 1's loads may be out); after the barrier
+    // for all, and all are done with chunk c - 1, whose buffer chunk c + 2 fills.
+    if (steady || c + 1 < chunks) __builtin_amdgcn_s_waitcnt(hx::kWaitVm0 | (kLtVT + XL));
+    else __builtin_amdgcn_s_waitcnt(hx::kWaitVm0);
+    // A plain barrier between compiler fences: __syncthreads would wait for chunk c + 1 too.
+    // This wave's reads of chunk c - 1 have returned, since its MFMAs used them.
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (steady || c + 2 < chunks) load(next, c + 2);
+    uint4 a[kLtVT];
+#pragma unroll
+    for (int v = 0; v < kLtVT; ++v)
+      a[v] = *reinterpret_cast<const uint4*>(cur.w + (kLtVT * w + v) * kLtTileBytes + frag);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const uint4 b = *reinterpret_cast<const uint4*>(cur.x + t * kLtTileBytes + frag);
+#pragma unroll
+      for (int v = 0; v < kLtVT; ++v)
+        acc[v][t] = hx::Elem<T>::mfma16x16x32(hx::as_v8<T>(a[v]), hx::as_v8<T>(b), acc[v][t]);
+    }
+  };
+  load(buf0, 0);
+  load(buf1, 1);  // hidden is a multiple of 128: at least four chunks
+  // In the steady loop every step loads, without a branch: on a path around a load the
+  // compiler would add a wait for all of them.
+  int c = 0;
+  for (; c + 4 < chunks; c += 3) {
+    step(c, buf0, buf2, true);
+    step(c + 1, buf1, buf0, true);
+    step(c + 2, buf2, buf1, true);
+  }
+  if (c < chunks) step(c, buf0, buf2, false);
+  if (c + 1 < chunks) step(c + 1, buf1, buf0, false);
+  if (c + 2 < chunks) step(c + 2, buf2, buf1, false);
+  if (c + 3 < chunks) step(c + 3, buf0, buf2, false);
+  __syncthreads();  // every wave is done with the chunks
+
+  uint64_t (*const s_key)[NT * 16] = reinterpret_cast<uint64_t (*)[NT * 16]>(&buf0);
+  static_assert(sizeof(uint64_t) * kLtWaves * NT * 16 <= sizeof(LtBuf<NT>), "the keys fit a chunk buffer");
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int tok = 16 * t + (lane & 15);
+    uint64_t best = 0;
+#pragma unroll
+    for (int v = 0; v < kLtVT; ++v) {
+      const int64_t vr0 = v0 + 16 * (kLtVT * w + v) + 4 * (lane >> 4);
+      best = max_u64(best, lg_finish<T>(acc[v][t], vr0, vocab, tok, n, logits, ld_logits));
+    }
+    best = max_u64(best, shfl_xor_u64(best, 16));
+    best = max_u64(best, shfl_xor_u64(best, 32));
+    if (lane < 16) s_key[w][16 * t + lane] = best;
+  }
+  __syncthreads();
+  for (int j = tid; j < n; j += kLtThreads) {
+    uint64_t m = s_key[0][j];
+#pragma unroll
+    for (int ww = 1; ww < kLtWaves; ++ww) m = max_u64(m, s_key[ww][j]);
     partial[(int64_t)j * tiles + hx::wg_x()] = m;
   }
 }
@@ -274,25 +415,42 @@ LogitsLayout logits_layout(int64_t n_rows, int64_t vocab, int32_t hidden) {
   return l;
 }
 
+// From kLtMinTiles row tiles on, and where its 640-row workgroups fill at least three quarters
+// of the rounds of one per CU that they take, the wide kernel. A call at 151936 x 2560 bf16
+// (norm, product, reduce; in us, with the logits written): 80 rows 168 (179) there against 160
+// (180) here, 100 rows 174 (186) against 180 (197), 129 rows 187 (199) against 200 (216), 160
+// rows 193 (207) against 213 (229). Row offsets within a workgroup are 32-bit: ld_emb below 2^20.
+constexpr int kLtMinTiles = 7;
+
+// Launches one group's product; returns its workgroups over the vocab (partial keys a row).
 template <typename T, int NT>
-void launch_argmax(int tiles, hipStream_t s, const uint16_t* emb, int64_t ld_emb, int64_t vocab,
+int launch_argmax(int tiles, hipStream_t s, const uint16_t* emb, int64_t ld_emb, int64_t vocab,
                    int hidden, const uint16_t* xn, int n, uint64_t* partial, uint16_t* logits,
                    int64_t ld_logits) {
+  if constexpr (NT >= kLtMinTiles) {
+    const int64_t wide = (vocab + kLtVocab - 1) / kLtVocab;
+    if (4 * wide >= 3 * ((wide + 255) / 256 * 256) && ld_emb < (int64_t)1 << 20) {
+      hipLaunchKernelGGL((logits_argmax_wide_kernel<T, NT>), dim3((unsigned)wide), dim3(kLtThreads), 0, s, emb, ld_emb,
+                         vocab, hidden, xn, n, (int32_t)wide, partial, logits, ld_logits);
+      return (int)wide;
+    }
+  }
   hipLaunchKernelGGL((logits_argmax_kernel<T, NT>), dim3(tiles), dim3(kLgThreads), 0, s, emb, ld_emb,
                      vocab, hidden, xn, n, tiles, partial, logits, ld_logits);
+  return tiles;
 }
 
 template <typename T>
-void launch_group(int nt, int tiles, hipStream_t s, const uint16_t* emb, int64_t ld_emb,
+int launch_group(int nt, int tiles, hipStream_t s, const uint16_t* emb, int64_t ld_emb,
                   int64_t vocab, int hidden, const uint16_t* xn, int n, uint64_t* partial,
                   uint16_t* logits, int64_t ld_logits) {
   switch (nt) {
 #define HX_LG_CASE(K) \
-  case K: launch_argmax<T, K>(tiles, s, emb, ld_emb, vocab, hidden, xn, n, partial, logits, ld_logits); break;
+  case K: return launch_argmax<T, K>(tiles, s, emb, ld_emb, vocab, hidden, xn, n, partial, logits, ld_logits);
     HX_LG_CASE(1) HX_LG_CASE(2) HX_LG_CASE(3) HX_LG_CASE(4) HX_LG_CASE(5)
     HX_LG_CASE(6) HX_LG_CASE(7) HX_LG_CASE(8) HX_LG_CASE(9) HX_LG_CASE(10)
 #undef HX_LG_CASE
-    default: break;
+    default: return tiles;
   }
 }
 
@@ -343,13 +501,14 @@ extern "C" int hx_final_norm_logits_argmax(
       hipLaunchKernelGGL(final_norm_kernel<_Float16>, dim3(pad), dim3(kLgThreads), 0, s, x, hidden_row_stride,
                          total_rows, logit_indices + r0, (int64_t)n, norm_weight, eps, (int)hidden, xn, ok);
     uint16_t* lg_group = lg != nullptr ? lg + r0 * logits_row_stride : nullptr;
+    int used;
     if (dtype == HX_DTYPE_BF16)
-      launch_group<__bf16>(pad / 16, lay.tiles, s, emb, embedding_row_stride, vocab, hidden, xn, n, partial,
+      used = launch_group<__bf16>(pad / 16, lay.tiles, s, emb, embedding_row_stride, vocab, hidden, xn, n, partial,
                            lg_group, logits_row_stride);
     else
-      launch_group<_Float16>(pad / 16, lay.tiles, s, emb, embedding_row_stride, vocab, hidden, xn, n, partial,
+      used = launch_group<_Float16>(pad / 16, lay.tiles, s, emb, embedding_row_stride, vocab, hidden, xn, n, partial,
                              lg_group, logits_row_stride);
-    hipLaunchKernelGGL(argmax_reduce_kernel, dim3(n), dim3(kLgThreads), 0, s, partial, lay.tiles, ok,
+    hipLaunchKernelGGL(argmax_reduce_kernel, dim3(n), dim3(kLgThreads), 0, s, partial, used, ok,
                        token_ids + r0, max_logits != nullptr ? max_logits + r0 : nullptr);
   }
   return hx::status_from_hip(hipGetLastError());

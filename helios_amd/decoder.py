@@ -90,6 +90,14 @@ class PagedQwen3Decoder:
             w.is_contiguous() and w.dtype == dtype and w.data_ptr() % 16 == 0 and w.shape[0] % 32 == 0
             and w.shape[1] % 64 == 0 for w in (layer["qkv"], layer["o"], layer["gate_up"], layer["down"]))
 
+    def _fused_heads(self, logit_indices: torch.Tensor, dtype: torch.dtype) -> bool:
+        """Whether the logits come from the fused heads kernel: one pass over the embedding
+        (up to 160 rows), in a layout it can read."""
+        w = self.embedding
+        return (logit_indices.numel() <= 160 and dtype in (torch.bfloat16, torch.float16) and w.dtype == dtype
+                and w.shape[1] % 128 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and self.final_norm.dtype == torch.float32)
+
     @torch.inference_mode()
     def forward_packed(self, input_ids: torch.Tensor, cache: PackedBatchCache, *,
                        fused_rope: bool = True, attention_events: list | None = None,
@@ -98,9 +106,9 @@ class PagedQwen3Decoder:
         argmax token ids (engine.py:470-473). ``attention_events`` collects (start, end)
         CUDA events around each layer's attention step.
 
-        With ``fused_rope`` (this build's sequence) the greedy ids come from the fused
-        final-norm / logits / argmax kernels and no logits are written; otherwise the
-        reference's logits are computed and ``argmax`` taken."""
+        With ``fused_rope`` (this build's sequence) the logits or greedy ids come from the
+        fused final-norm / logits / argmax kernels (no logits are written for the ids);
+        otherwise the reference's logits are computed and ``argmax`` taken."""
         config = self.config
         if input_ids.shape != (1, sum(cache.counts)):
             raise ValueError(f"input_ids must be [1, {sum(cache.counts)}]: one token per packed row of the tick.")
@@ -159,6 +167,10 @@ class PagedQwen3Decoder:
         if greedy and fused_rope:
             return ops.final_norm_logits_argmax(x, cache.logit_indices, self.final_norm, self.embedding,
                                                 eps).token_ids
+        if fused_rope and self._fused_heads(cache.logit_indices, x.dtype):
+            logits = ops.final_norm_logits_argmax(x, cache.logit_indices, self.final_norm, self.embedding, eps,
+                                                  return_logits=True).logits
+            return logits
         x = x.index_select(1, cache.logit_indices)
         logits = (_rms_norm(x, self.final_norm, eps).to(config.dtype) @ self.embedding.t())[0]
         return logits.argmax(dim=-1) if greedy else logits

@@ -74,6 +74,28 @@ def test_matches_oracle(device, dtype, picks):
     np.testing.assert_array_equal(res.max_logits.cpu().numpy(), got.max(axis=-1))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("picks", [97, 113, 129, 160])
+def test_many_rows_over_640_row_vocab_tiles(device, picks, dtype):
+    """The kernel for seven and more row tiles, which needs a vocab that fills the chip: 199
+    workgroups of 640 rows, the last of them 29 rows, hidden of five buffer turns and a
+    rest. Against fp32 products of the same normalised rows, every logit and pick."""
+    say("logits many rows", picks, dtype)
+    hidden, vocab = 512, 198 * 640 + 29
+    x, w, emb, idx = _inputs(device, 200, hidden, vocab, picks, seed=picks, std=0.03)
+    x, emb = x.to(dtype), emb.to(dtype)
+    res = ops.final_norm_logits_argmax(x, idx, w, emb, 1e-6, return_logits=True)
+    few = [ops.final_norm_logits_argmax(x, part, w, emb, 1e-6, return_logits=True) for part in idx.split(16)]
+    torch.cuda.synchronize()
+    got, want = res.logits.float(), torch.cat([f.logits for f in few]).float()
+    # The few-row kernel adds the same fp32 products in another order: at most one rounding
+    # step apart (plus the sums' own error near zero), and rarely that.
+    ulp = BF16_ULP if dtype == torch.bfloat16 else BF16_ULP / 8
+    assert ((got - want).abs() <= ulp * want.abs() + 1e-5).all()
+    assert (got != want).float().mean() < 2e-2
+    assert torch.equal(res.token_ids, got.argmax(dim=-1)) and torch.equal(res.max_logits, got.max(dim=-1).values)
+
+
 def test_ties_and_planted_winners(device):
     say("logits ties")
     rows, hidden, vocab = 8, 384, 777  # vocab tail: 777 = 6 x 128 + 9
