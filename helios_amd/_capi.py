@@ -6,6 +6,7 @@ Loading fails loudly: there is no CPU or PyTorch fallback for any operation.
 from __future__ import annotations
 
 import ctypes
+import struct
 from pathlib import Path
 
 LIBRARY_PATH = Path(__file__).resolve().with_name("libhelios_paged.so")
@@ -72,6 +73,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          _i32, _i32, _i32, _i32, _i32, _i32, _i32,
          _c_void_p, _size, _c_void_p],
     ),
+    "hx_varlen_attn_call": (ctypes.c_int, [ctypes.c_char_p, _c_void_p]),
     "hx_varlen_attn_run": (
         ctypes.c_int,
         [_c_void_p, _i64, _i64,
@@ -220,6 +222,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
          _c_void_p, _size, _c_void_p],
     ),
 }
+
+# hx_attn_call: 8-byte integers and addresses, one double (the scale).
+ATTN_CALL = struct.Struct("<19qd20q")
 
 _lib: ctypes.CDLL | None = None
 

@@ -3392,6 +3392,33 @@ int hx_varlen_attn_append_run(const void* q, int64_t q_row_stride, int64_t q_hea
                   combine_seqs_hint, workspace, workspace_bytes, stream, &app);
 }
 
+int hx_varlen_attn_call(const hx_attn_call* call, void* stream) {
+  if (call == nullptr || call->size != (int64_t)sizeof(hx_attn_call)) return HX_E_INVALID_ARG;
+  const hx_attn_call& c = *call;
+  for (const int64_t v : {c.num_pages, c.page_size, c.block_table_stride, c.batch, c.total_q, c.max_q, c.max_k,
+                          c.n_q_heads, c.n_kv_heads, c.head_dim, c.window_left, c.window_right, c.dtype,
+                          c.decode_items_hint, c.prefill_items_hint, c.combine_seqs_hint})
+    if (v < INT32_MIN || v > INT32_MAX) return HX_E_INVALID_ARG;
+  if (c.workspace_bytes < 0) return HX_E_INVALID_ARG;
+  AppendSpec app;
+  app.k_new = c.k_new;
+  app.v_new = c.v_new;
+  app.kn_row = c.k_new_row_stride;
+  app.kn_head = c.k_new_head_stride;
+  app.vn_row = c.v_new_row_stride;
+  app.vn_head = c.v_new_head_stride;
+  app.write_slots = c.write_slots;
+  app.pool_rows = c.pool_rows;
+  return run_impl(c.q, c.q_row_stride, c.q_head_stride, nullptr, 0, c.k_cache, c.v_cache, c.kv_row_stride,
+                  c.kv_head_stride, (int32_t)c.num_pages, (int32_t)c.page_size, c.block_table,
+                  (int32_t)c.block_table_stride, (int32_t)c.batch, (int32_t)c.total_q, (int32_t)c.max_q,
+                  (int32_t)c.max_k, (int32_t)c.n_q_heads, (int32_t)c.n_kv_heads, (int32_t)c.head_dim, (float)c.scale,
+                  (int32_t)c.window_left, (int32_t)c.window_right, (int32_t)c.dtype, c.out, c.o_row_stride,
+                  c.o_head_stride, c.lse, (int32_t)c.decode_items_hint, (int32_t)c.prefill_items_hint,
+                  (int32_t)c.combine_seqs_hint, c.workspace, (size_t)c.workspace_bytes, stream,
+                  c.k_new != nullptr ? &app : nullptr);
+}
+
 int hx_varlen_attn(const void* q, int64_t q_row_stride, int64_t q_head_stride,
                    const void* k_cache, const void* v_cache,
                    int64_t kv_row_stride, int64_t kv_head_stride,

@@ -194,13 +194,7 @@ def qk_norm_rope_append(
     if queries.dtype != keys.dtype or queries.stride(2) != 1:
         raise ValueError("queries must share the K/V dtype and have a contiguous head_dim.")
     head_dim = queries.shape[2]
-    for name, w in (("q_norm_weight", q_norm_weight), ("k_norm_weight", k_norm_weight)):
-        if w.dtype != torch.float32 or w.numel() != head_dim or not w.is_contiguous():
-            raise ValueError(f"{name} must be a contiguous float32 [head_dim] tensor.")
-    if (cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.shape != sin.shape
-            or cos.ndim != 2 or cos.shape[1] != head_dim or not cos.is_contiguous()
-            or not sin.is_contiguous()):
-        raise ValueError("cos/sin must be contiguous float32 [rows, head_dim] tables.")
+    _check_rope(q_norm_weight, k_norm_weight, cos, sin, head_dim)
     positions = positions.reshape(-1)
     if positions.dtype != torch.int64 or positions.numel() != queries.shape[0]:
         raise ValueError("positions must be int64 with one entry per row.")
@@ -226,6 +220,56 @@ def qk_norm_rope_append(
         _stream_ptr(device),
     )
     _capi.check(code, "hx_qk_norm_rope_append")
+    return out
+
+
+def _check_rope(q_norm_weight, k_norm_weight, cos, sin, head_dim: int) -> None:
+    """Checks of the norm weights and RoPE tables."""
+    for name, w in (("q_norm_weight", q_norm_weight), ("k_norm_weight", k_norm_weight)):
+        if w.dtype != torch.float32 or w.numel() != head_dim or not w.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous float32 [head_dim] tensor.")
+    if (cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.shape != sin.shape
+            or cos.ndim != 2 or cos.shape[1] != head_dim or not cos.is_contiguous()
+            or not sin.is_contiguous()):
+        raise ValueError("cos/sin must be contiguous float32 [rows, head_dim] tables.")
+
+
+def qk_norm_rope_append_packed(
+    queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, n_q_heads: int, q_norm_weight: torch.Tensor,
+    k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor,
+    k_cache: torch.Tensor, v_cache: torch.Tensor, write_slots: torch.Tensor, eps: float,
+) -> torch.Tensor | None:
+    """``qk_norm_rope_append`` for projections as they come, queries ``[1, T, Hq * d]`` and
+    keys / values ``[1, T, Hkv * d]`` (any row stride, contiguous heads), contiguous pools
+    and index vectors, without making row views on the way: the same launch. None, and
+    nothing launched, for any other layout, type or device."""
+    dtype, index = queries.dtype, queries.get_device()
+    code = _SUPPORTED.get(dtype)
+    if code is None or index < 0 or queries.ndim != 3 or keys.ndim != 3 or k_cache.ndim != 4:
+        return None
+    one, rows, width = queries.shape
+    n_kv, head_dim = k_cache.shape[2], k_cache.shape[3]
+    if (one != 1 or width != n_q_heads * head_dim or keys.shape != (1, rows, n_kv * head_dim)
+            or values.shape != keys.shape or keys.dtype is not dtype or values.dtype is not dtype
+            or queries.stride(2) != 1 or keys.stride(2) != 1 or values.stride(2) != 1
+            or k_cache.dtype is not dtype or v_cache.dtype is not dtype or v_cache.shape != k_cache.shape
+            or not k_cache.is_contiguous() or not v_cache.is_contiguous()
+            or write_slots.dtype is not torch.int64 or write_slots.ndim != 1 or write_slots.numel() != rows
+            or positions.dtype is not torch.int64 or positions.ndim != 1 or positions.numel() != rows
+            or not write_slots.is_contiguous() or not positions.is_contiguous()):
+        return None
+    for t in (keys, values, q_norm_weight, k_norm_weight, cos, sin, positions, k_cache, v_cache, write_slots):
+        if t.get_device() != index:
+            return None
+    _check_rope(q_norm_weight, k_norm_weight, cos, sin, head_dim)
+    out = torch.empty((rows, n_q_heads, head_dim), dtype=dtype, device=queries.device)
+    status = _capi.lib().hx_qk_norm_rope_append(
+        queries.data_ptr(), queries.stride(1), head_dim, keys.data_ptr(), keys.stride(1), head_dim,
+        values.data_ptr(), values.stride(1), head_dim, q_norm_weight.data_ptr(), k_norm_weight.data_ptr(),
+        cos.data_ptr(), sin.data_ptr(), cos.shape[0], positions.data_ptr(), rows, n_q_heads, n_kv, head_dim, eps, code,
+        out.data_ptr(), width, head_dim, k_cache.data_ptr(), v_cache.data_ptr(), k_cache.shape[0] * k_cache.shape[1],
+        write_slots.data_ptr(), torch._C._cuda_getCurrentRawStream(index))
+    _capi.check(status, "hx_qk_norm_rope_append")
     return out
 
 
@@ -670,6 +714,14 @@ class VarlenAttnPlan:
             self.hints = count_items(q_lens, k_lens, n_q_heads, n_kv_heads, window)
         else:
             self.hints = (-1, -1, -1)
+        # What append_attend compares its tensors with.
+        self._scale = 1.0 / math.sqrt(head_dim)
+        self._q_shape = torch.Size((1, n_q_heads, total_q, head_dim))
+        self._kv_shape = torch.Size((1, n_kv_heads, total_q, head_dim))
+        self._page_shape = torch.Size((page_size, n_kv_heads, head_dim))
+        self._page_stride = (page_size * n_kv_heads * head_dim, n_kv_heads * head_dim, head_dim, 1)
+        self._table_shape = torch.Size((max(batch, 0), block_table_stride))
+        self._out_stride = (n_q_heads * head_dim, head_dim, n_q_heads * head_dim, 1)
         cu_q, cu_k, used = self._metadata
         code = _capi.lib().hx_varlen_attn_plan(
             cu_q.data_ptr(),
@@ -691,6 +743,81 @@ class VarlenAttnPlan:
         word = self.error_word()
         if word:
             raise RuntimeError(f"paged attention metadata error {word:#x}: {describe_error_word(word)}")
+
+    def append_attend(self, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor,
+                      k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
+                      write_slots: torch.Tensor) -> torch.Tensor | None:
+        """``run(append=...)`` of one layer for the layout the decoder's projections have:
+        queries ``[1, Hq, total_q, d]``, keys / values ``[1, Hkv, total_q, d]`` (any row and
+        head strides), contiguous pools; returns ``[1, Hq, total_q, d]`` (packed rows in
+        memory), without making row views on the way. The same launches and bits. None, and
+        nothing launched, for any other layout, type or device: the caller then takes ``run``.
+
+        A short tick's call is bound by this host path. 1 request of 300 keys: 26.4 us a
+        call through the row views and ``run``."""
+        dtype, index = queries.dtype, self.device.index
+        code = _SUPPORTED.get(dtype)
+        if (code is None or CHECK_ERRORS or self.page_size <= 0
+                or queries.shape != self._q_shape or keys.shape != self._kv_shape or values.shape != self._kv_shape
+                or keys.dtype is not dtype or values.dtype is not dtype
+                or k_cache.dtype is not dtype or v_cache.dtype is not dtype
+                or k_cache.ndim != 4 or k_cache.shape[1:] != self._page_shape or v_cache.shape != k_cache.shape
+                or k_cache.stride() != self._page_stride or v_cache.stride() != self._page_stride
+                or block_table.dtype is not torch.int32 or block_table.shape != self._table_shape
+                or block_table.stride() != (self.block_table_stride, 1)
+                or write_slots.dtype is not torch.int64 or write_slots.ndim != 1
+                or write_slots.numel() != self.total_q or write_slots.stride(0) != 1
+                or queries.get_device() != index or keys.get_device() != index or values.get_device() != index
+                or k_cache.get_device() != index or v_cache.get_device() != index
+                or block_table.get_device() != index or write_slots.get_device() != index):
+            return None
+        qs, ks, vs = queries.stride(), keys.stride(), values.stride()
+        q_ptr, k_ptr, v_ptr = queries.data_ptr(), keys.data_ptr(), values.data_ptr()
+        # 16-byte loads of the new rows, and of q (whose run raises otherwise).
+        if (qs[3] != 1 or ks[3] != 1 or vs[3] != 1 or (q_ptr | k_ptr | v_ptr) & 15
+                or (qs[1] | qs[2] | ks[1] | ks[2] | vs[1] | vs[2]) & 7):
+            return None
+        pages, page_size, heads, dim = k_cache.shape
+        out = torch.empty_strided(self._q_shape, self._out_stride, dtype=dtype, device=self.device)
+        status = _capi.lib().hx_varlen_attn_call(_capi.ATTN_CALL.pack(
+            _capi.ATTN_CALL.size, q_ptr, qs[2], qs[1], k_cache.data_ptr(), v_cache.data_ptr(), heads * dim, dim,
+            pages, page_size, block_table.data_ptr(), self.block_table_stride,
+            self.batch, self.total_q, self.max_q, self.max_k, self.n_q_heads, heads, dim,
+            self._scale, self.window[0], self.window[1], code, out.data_ptr(), self._out_stride[0], dim, 0,
+            k_ptr, ks[2], ks[1], v_ptr, vs[2], vs[1], write_slots.data_ptr(), pages * page_size,
+            *self.hints, self.ws_ptr, self.ws_bytes), torch._C._cuda_getCurrentRawStream(index))
+        _capi.check(status, "hx_varlen_attn_call")
+        return out
+
+    def attend_rows(self, query: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                    block_table: torch.Tensor) -> torch.Tensor | None:
+        """``run(query, ...)`` without its options, for contiguous packed queries
+        ``[total_q, Hq, d]`` and contiguous pools; None, and nothing launched, otherwise."""
+        dtype, index = query.dtype, self.device.index
+        code = _SUPPORTED.get(dtype)
+        if (code is None or CHECK_ERRORS or self.page_size <= 0
+                or query.ndim != 3 or query.shape[0] != self.total_q or query.shape[1] != self.n_q_heads
+                or query.shape[2] != self.head_dim or not query.is_contiguous()
+                or k_cache.dtype is not dtype or v_cache.dtype is not dtype
+                or k_cache.ndim != 4 or k_cache.shape[1:] != self._page_shape or v_cache.shape != k_cache.shape
+                or k_cache.stride() != self._page_stride or v_cache.stride() != self._page_stride
+                or block_table.dtype is not torch.int32 or block_table.shape != self._table_shape
+                or block_table.stride() != (self.block_table_stride, 1)
+                or query.get_device() != index or k_cache.get_device() != index or v_cache.get_device() != index
+                or block_table.get_device() != index):
+            return None
+        pages, page_size, heads, dim = k_cache.shape
+        row = self._out_stride[0]
+        out = torch.empty_like(query)
+        status = _capi.lib().hx_varlen_attn_call(_capi.ATTN_CALL.pack(
+            _capi.ATTN_CALL.size, query.data_ptr(), row, dim, k_cache.data_ptr(), v_cache.data_ptr(), heads * dim, dim,
+            pages, page_size, block_table.data_ptr(), self.block_table_stride,
+            self.batch, self.total_q, self.max_q, self.max_k, self.n_q_heads, heads, dim,
+            self._scale, self.window[0], self.window[1], code, out.data_ptr(), row, dim, 0,
+            0, 0, 0, 0, 0, 0, 0, 0, *self.hints, self.ws_ptr, self.ws_bytes),
+            torch._C._cuda_getCurrentRawStream(index))
+        _capi.check(status, "hx_varlen_attn_call")
+        return out
 
     def run(
         self,

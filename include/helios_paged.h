@@ -343,6 +343,40 @@ int hx_varlen_attn(const void* q, int64_t q_row_stride, int64_t q_head_stride,
                    float* lse,
                    void* workspace, size_t workspace_bytes, void* stream);
 
+/* hx_varlen_attn_run / hx_varlen_attn_append_run (k_new not NULL) with the arguments in one
+ * struct of 8-byte fields, which a caller of many short calls can fill in one step. The
+ * fields are those functions' arguments. size is sizeof(hx_attn_call) (HX_E_INVALID_ARG
+ * otherwise, and for a field outside its argument's range). */
+typedef struct hx_attn_call {
+  int64_t size;
+  const void* q;
+  int64_t q_row_stride, q_head_stride;
+  const void* k_cache;
+  const void* v_cache;
+  int64_t kv_row_stride, kv_head_stride;
+  int64_t num_pages, page_size;
+  const int32_t* block_table;
+  int64_t block_table_stride;
+  int64_t batch, total_q, max_q, max_k;
+  int64_t n_q_heads, n_kv_heads, head_dim;
+  double scale;
+  int64_t window_left, window_right;
+  int64_t dtype;
+  void* out;
+  int64_t o_row_stride, o_head_stride;
+  float* lse;
+  const void* k_new;
+  int64_t k_new_row_stride, k_new_head_stride;
+  const void* v_new;
+  int64_t v_new_row_stride, v_new_head_stride;
+  const int64_t* write_slots;
+  int64_t pool_rows;
+  int64_t decode_items_hint, prefill_items_hint, combine_seqs_hint;
+  void* workspace;
+  int64_t workspace_bytes;
+} hx_attn_call;
+int hx_varlen_attn_call(const hx_attn_call* call, void* stream);
+
 /* Byte offset of the int32 error word inside the workspace (OR of HX_WERR_* bits,
  * cleared by each hx_varlen_attn_plan). */
 size_t hx_varlen_attn_error_word_offset(void);
