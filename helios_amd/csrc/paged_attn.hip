@@ -2166,8 +2166,10 @@ __global__ __launch_bounds__(kChunkThreads, 2) void chunk_pair_kernel(RunArgs a0
 // element type and the remainder (17 bits or more of p), and the splits' partial results
 // stay in fp32. q . k is exact products in fp32 sums.
 // Bound by latency at these sizes. 24 decode rows of 200-2048 keys and chunks of 512 and
-// 333 rows, 16/4 heads, d = 64: 19.5 us and 4.8 us for the merge; scores and P V on the VALU,
-// 16 units a workgroup and no splits, took 284 us.
+// 333 rows, 16/4 heads, d = 64: 18.6 us and 4.8 us for the merge; scores and P V on the VALU,
+// 16 units a workgroup and no splits, took 284 us. Two tiles in flight instead of one gained
+// nothing. Workgroups per CU by padded head dim (the launch bounds): at 128 a third and at 256 a
+// second one (chunks of 600 rows at 256: 107.6 -> 89.6 us a call; at 96 a third lost 5 %).
 constexpr int kWideUnits = 64;   // units of a chunk block: 4 waves x 16
 constexpr int kWideDecUnits = 16;
 constexpr int kWideThreads = 256;
@@ -2353,17 +2355,22 @@ __device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws,
         s[kb] = E::mfma16x16x32(hx::as_v8<T>(kf), hx::as_v8<T>(qf[st]), s[kb]);
       }
     const int key_base = t * kTile + (DEC ? 16 * w : 0) + 4 * gg;  // of s[0][0]
+    // Masked only where some lane's keys are not all visible (a wave-uniform test).
+    if (__any(key_base < klo || key_base + 16 * (NB - 1) + 3 > khi)) {
+#pragma unroll
+      for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = key_base + 16 * kb + i;
+          s[kb][i] = key >= klo && key <= khi ? s[kb][i] : -INFINITY;
+        }
+    }
     float mt = -INFINITY;
 #pragma unroll
     for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = key_base + 16 * kb + i;
-        const float x = key >= klo && key <= khi ? s[kb][i] * a.scale_log2 : -INFINITY;
-        s[kb][i] = x;
-        mt = fmaxf(mt, x);
-      }
-    mt = fmaxf(m, hx::max_xor32(hx::max_xor16(mt)));
+      for (int i = 0; i < 4; ++i) mt = fmaxf(mt, s[kb][i]);
+    mt = fmaxf(m, hx::max_xor32(hx::max_xor16(mt)) * a.scale_log2);  // the scale is positive
     if (__any(mt > m)) {
       const float alpha = m == -INFINITY ? 0.f : hx::fast_exp2(m - mt);  // nothing summed yet: any factor will do
       l *= alpha;
@@ -2377,7 +2384,7 @@ __device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws,
     for (int kb = 0; kb < NB; ++kb) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        s[kb][i] = hx::fast_exp2(s[kb][i] + neg_m);  // -inf -> 0
+        s[kb][i] = hx::fast_exp2(fmaf(s[kb][i], a.scale_log2, neg_m));  // -inf -> 0
         l += s[kb][i];
       }
     }
@@ -2502,7 +2509,7 @@ __device__ __forceinline__ bool wide_plan_ok(const RunArgs& a, const WideShape& 
 // Workgroups: n_wg of them (the launch's count). Every loop bound comes from the plan
 // header and is the same for the whole workgroup.
 template <typename T, int DP>
-__global__ __launch_bounds__(kWideThreads, DP <= 64 ? 4 : DP <= 128 ? 2 : 1) void wide_kernel(RunArgs a, WideShape ws, int n_wg) {
+__global__ __launch_bounds__(kWideThreads, DP <= 64 ? 4 : DP == 128 ? 3 : 2) void wide_kernel(RunArgs a, WideShape ws, int n_wg) {
   __shared__ WideLds<DP> lds;
   int4 counts;
   bool lists;
