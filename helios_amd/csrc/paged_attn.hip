@@ -363,6 +363,7 @@ __device__ void write_plan_header(const PlanArgs& a, int err, int4 totals) {
 
 // The planner's serial form: one thread walks each sequence's row blocks in every pass.
 // Used when the chunk sequences or their row blocks exceed the LDS lists of plan_kernel.
+template <int TH>
 __device__ void plan_serial(const PlanArgs& a, int* wave_tot, int* err_bits, int4* totals) {
   int err = 0;
 
@@ -372,7 +373,7 @@ __device__ void plan_serial(const PlanArgs& a, int* wave_tot, int* err_bits, int
   if (hx::tid_x() == 0) max_blk_tiles = 0;
   __syncthreads();
   int64_t pf_items0 = 0, pf_tiles = 0;
-  for (int b0 = 0; b0 < a.batch; b0 += kPlanThreads) {
+  for (int b0 = 0; b0 < a.batch; b0 += TH) {
     const int b = b0 + hx::tid_x();
     int items = 0, tiles = 0, tmax = 0;
     if (b < a.batch) {
@@ -400,7 +401,7 @@ __device__ void plan_serial(const PlanArgs& a, int* wave_tot, int* err_bits, int
   // runs it the same number of times, since the search depends only on block totals).
   auto chunk_wgs = [&](int st) -> int64_t {
     int64_t total = 0;
-    for (int b0 = 0; b0 < a.batch; b0 += kPlanThreads) {
+    for (int b0 = 0; b0 < a.batch; b0 += TH) {
       const int b = b0 + hx::tid_x();
       int wg = 0;
       if (b < a.batch) {
@@ -426,7 +427,7 @@ __device__ void plan_serial(const PlanArgs& a, int* wave_tot, int* err_bits, int
 
   // Pass 2: work lists.
   int base_dec = 0, base_pf = 0, base_comb = 0, base_slot = 0;
-  for (int b0 = 0; b0 < a.batch; b0 += kPlanThreads) {
+  for (int b0 = 0; b0 < a.batch; b0 += TH) {
     const int b = b0 + hx::tid_x();
     const bool active = b < a.batch;
     SeqMeta m{0, 0, 0, 0};
@@ -583,14 +584,21 @@ constexpr int kPlanChunkSeqs = 1024;
 constexpr int kPlanBlocks = 4096;
 constexpr int kPlanSearchWork = 1 << 16;  // candidates x blocks evaluated in one pass
 constexpr int kPlanSortBlocks = 256;
-static_assert(3 * kPlanSortBlocks <= kPlanThreads, "sort keys, item counts and ranks share the search buffer");
-static_assert(4 * kPlanSortBlocks <= kPlanThreads, "at least four threads rank each block");
+// Ticks of at most 256 sequences and 96 blocks take 256 threads: every pass ends in barriers
+// and per-wave totals, and four waves get through them sooner than sixteen (64 decode rows
+// 5.6 -> 3.9 us; 14, 64 and 76 blocks 12.3 -> 9.4, 9.7 -> 7.7 and 13.3 -> 12.0 us; 126 blocks
+// would be slower).
+constexpr int kPlanSmallThreads = 256;
+constexpr int kPlanSmallBlocks = 96;
+constexpr int kPlanOwnItems = 32;  // decode items a row's own thread writes
+static_assert(kPlanSortBlocks <= kPlanSmallThreads, "a thread per sorted block");
 
-__global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
-  __shared__ int wave_tot[kPlanThreads / 64];
+template <int TH>
+__global__ __launch_bounds__(TH) void plan_kernel(PlanArgs a) {
+  __shared__ int wave_tot[TH / 64];
   __shared__ WaveTotals wt;
   __shared__ int err_bits;
-  __shared__ int cand_wgs[kPlanThreads];  // split-size search: workgroups per candidate
+  __shared__ int cand_wgs[TH > 3 * kPlanSortBlocks ? TH : 3 * kPlanSortBlocks];  // split-size search: workgroups per candidate
   __shared__ int best_st, best_one;
   // Chunk sequence k: its sequence index, first row, clamped (n, L), first flat block, and its item /
   // combine-record / partial-slot offsets once known.
@@ -609,7 +617,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   int err = 0;
   if (a.plain) {
     __syncthreads();
-    for (int b = tid; b < a.batch; b += kPlanThreads) {
+    for (int b = tid; b < a.batch; b += TH) {
       const SeqMeta m = plan_seq(a, b, err);
       a.seq_info[b] = make_int4(m.q0, m.n, m.L, m.kvb);
     }
@@ -625,7 +633,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   int n_cs = 0, n_blk = 0;
   SeqMeta m_kept{0, 0, 0, 0};
   int k_kept = 0;
-  for (int b0 = 0; b0 < a.batch; b0 += kPlanThreads) {
+  for (int b0 = 0; b0 < a.batch; b0 += TH) {
     const int b = b0 + tid;
     SeqMeta m{0, 0, 0, 0};
     if (b < a.batch) m = plan_seq(a, b, err);
@@ -649,7 +657,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   }
   if (n_cs > kPlanChunkSeqs || n_blk > kPlanBlocks) {
     int4 totals;
-    plan_serial(a, wave_tot, &err_bits, &totals);
+    plan_serial<TH>(a, wave_tot, &err_bits, &totals);
     if (err) atomicOr(&err_bits, err);
     __syncthreads();
     if (tid == 0) write_plan_header(a, err_bits, totals);
@@ -676,7 +684,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   int2 tm = make_int2(0, 0);
   if (n_blk > 0) {
     int my_tiles = 0, my_max = 0;
-    for (int i = tid; i < n_blk; i += kPlanThreads) {
+    for (int i = tid; i < n_blk; i += TH) {
       int k, blk;
       block_of(i, k, blk);
       int tb, te;
@@ -696,18 +704,18 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   // evaluated at once (one per thread) and the smallest fitting one taken.
   auto chunk_wgs = [&](int st) -> int64_t {
     int wg = 0;
-    for (int i = tid; i < n_blk; i += kPlanThreads) wg += chunk_split_count(fb_tiles[i], st);
+    for (int i = tid; i < n_blk; i += TH) wg += chunk_split_count(fb_tiles[i], st);
     return (int64_t)block_sum_max(wg, 0, wt, turn).x * a.head_quads * a.hkv;
   };
   const int st0 = chunk_split_tiles(pf_tiles, pf_items0, a.hkv);
   int split_tiles = st0;
   if (st0 > 0 && tm.y > st0) {
     const int ncand = tm.y - st0;  // candidates st0 + 1 .. max tiles
-    if (ncand < kPlanThreads && (int64_t)(ncand + 1) * n_blk <= kPlanSearchWork) {
+    if (ncand < TH && (int64_t)(ncand + 1) * n_blk <= kPlanSearchWork) {
       // Workgroups at split size st0 + j for every j <= ncand, the blocks dealt over as many
       // threads as there are per candidate (one thread walking all blocks took 0.08 us a
       // block); the smallest fitting candidate wins an LDS atomicMin.
-      const int parts = kPlanThreads / (ncand + 1);
+      const int parts = TH / (ncand + 1);
       const int part = tid / (ncand + 1), j = tid - part * (ncand + 1);
       if (tid <= ncand) cand_wgs[tid] = 0;
       __syncthreads();
@@ -743,7 +751,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   // combine records (one per kCombRows split rows); exclusive scans in flat order.
   if (n_blk > 0) {
     int base_p = 0, base_c = 0, base_s = 0;
-    for (int i0 = 0; i0 < n_blk; i0 += kPlanThreads) {
+    for (int i0 = 0; i0 < n_blk; i0 += TH) {
       const int i = i0 + tid;
       int4 v = make_int4(0, 0, 0, 0);
       if (i < n_blk) {
@@ -779,11 +787,11 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
   // Phase 4: per sequence, item counts and offsets; decode items and sequence info.
   int base_dec = 0, base_pf = 0, base_comb = 0, base_slot = 0;
   int kc = 0;  // chunk sequences before this b0 round
-  for (int b0 = 0; b0 < a.batch; b0 += kPlanThreads) {
+  for (int b0 = 0; b0 < a.batch; b0 += TH) {
     const int b = b0 + tid;
     const bool active = b < a.batch;
     SeqMeta m = m_kept;
-    if (active && a.batch > kPlanThreads) m = plan_seq(a, b, err);
+    if (active && a.batch > TH) m = plan_seq(a, b, err);
     const int is_chunk = active && m.n >= 2;
     int4 cnt = make_int4(0, 0, 0, 0);  // decode items, chunk items, combine records, slots
     int s_first = 0, splits = 0;
@@ -794,7 +802,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
     }
     // The chunk sequence index of b: the same compaction as phase 0.
     int k = k_kept;
-    if (n_cs > 0 && a.batch > kPlanThreads) {
+    if (n_cs > 0 && a.batch > TH) {
       int4 ctot;
       k = kc + block_exclusive_scan4(make_int4(is_chunk, 0, 0, 0), wt, turn, &ctot).x;
       kc += ctot.x;
@@ -811,7 +819,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
     const int off_c = base_comb + pre.z, off_s = base_slot + pre.w;
     if (active) {
       a.seq_info[b] = make_int4(m.q0, m.n, m.L, m.kvb);
-      for (int j = 0; j < cnt.x; ++j) {
+      for (int j = 0; j < min(cnt.x, kPlanOwnItems); ++j) {
         if (off_d + j < a.max_dec) a.dec_items[off_d + j] = make_int4(b, s_first + j, m.q0, m.L);
       }
       if (cnt.z && m.n == 1 && off_c < a.max_comb) a.comb_seqs[off_c] = make_int4(b, off_d, splits, m.q0);
@@ -820,6 +828,17 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
         cs_off_c[k] = off_c;
         cs_off_s[k] = off_s;
       }
+    }
+    // The rest of a long row's decode items by its whole wave, row by row: one thread takes
+    // about 0.06 us an item (8 rows of 128 splits: 12.7 us of planning), a row's turn of the
+    // wave about 0.13 us.
+    for (uint64_t longer = __ballot(cnt.x > kPlanOwnItems); longer != 0; longer &= longer - 1) {
+      const int l = __builtin_ctzll(longer);
+      const int n_l = __builtin_amdgcn_readlane(cnt.x, l), o_l = __builtin_amdgcn_readlane(off_d, l);
+      const int4 it = make_int4(b0 + (tid & ~63) + l, __builtin_amdgcn_readlane(s_first, l),
+                                __builtin_amdgcn_readlane(m.q0, l), __builtin_amdgcn_readlane(m.L, l));
+      for (int j = kPlanOwnItems + (tid & 63); j < n_l; j += 64)
+        if (o_l + j < a.max_dec) a.dec_items[o_l + j] = make_int4(it.x, it.y + j, it.z, it.w);
     }
     base_dec += tot.x;
     base_pf += tot.y;
@@ -847,23 +866,21 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanArgs a) {
       blk_items[tid] = S * a.head_quads;
     }
     __syncthreads();
-    // 16 threads rank each block (4 when there are more than 64 blocks): items of the
-    // blocks that go before it.
-    const int sh = n_blk <= kPlanThreads / 16 ? 4 : 2;
-    const int i = tid >> sh;
-    int before = 0;
-    if (i < n_blk) {
+    // 16 threads rank each block (4 when there are many): items of the blocks before it.
+    const int sh = n_blk <= TH / 16 ? 4 : 2;
+    for (int i = tid >> sh; i < n_blk; i += TH >> sh) {
       const int key = blk_key[i];
+      int before = 0;
       for (int j = tid & ((1 << sh) - 1); j < n_blk; j += 1 << sh) {
         const int kj = blk_key[j];
         before += kj > key || (kj == key && j < i) ? blk_items[j] : 0;
       }
+      for (int m = 1; m < (1 << sh); m <<= 1) before += __shfl_xor(before, m);
+      if ((tid & ((1 << sh) - 1)) == 0) blk_first[i] = before;
     }
-    for (int m = 1; m < (1 << sh); m <<= 1) before += __shfl_xor(before, m);
-    if (i < n_blk && (tid & ((1 << sh) - 1)) == 0) blk_first[i] = before;
     __syncthreads();
   }
-  for (int i = tid; i < n_blk; i += kPlanThreads) {
+  for (int i = tid; i < n_blk; i += TH) {
     int k, blk;
     block_of(i, k, blk);
     const int f0 = cs_first[k];
@@ -2890,7 +2907,13 @@ int hx_varlen_attn_plan(const int32_t* cu_seq_q, const int32_t* cu_seq_k,
   a.win_right = window_right;
   a.hq = n_q_heads;
   a.hkv = n_kv_heads;
-  hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, static_cast<hipStream_t>(stream), a);
+  // Blocks of all chunks: at most one per rows_per_item rows, and one more per sequence.
+  const int64_t blocks = max_q >= 2 ? total_q / geo.rows_per_item + batch : 0;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (batch <= kPlanSmallThreads && blocks <= kPlanSmallBlocks)
+    hipLaunchKernelGGL((plan_kernel<kPlanSmallThreads>), dim3(1), dim3(kPlanSmallThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((plan_kernel<kPlanThreads>), dim3(1), dim3(kPlanThreads), 0, s, a);
   return hx::status_from_hip(hipGetLastError());
 }
 

@@ -108,3 +108,17 @@ def test_plan_lists_past_the_list_capacities(device):
     q_lens = [4160] * 64 + [1] * 3
     k_lens = [4160] * 64 + [300, 5000, 9000]
     _check("4160 blocks", q_lens, k_lens, device=device)
+
+
+@pytest.mark.parametrize("batch,chunk", [(1, 0), (256, 0), (257, 0), (3, 4096), (3, 4288), (40, 3600)])
+def test_plan_lists_around_the_small_planner(device, batch, chunk):
+    """256 threads up to 256 sequences and 96 blocks, 1024 beyond; rows of 32 and 33 decode
+    items, where the wave takes over from the row's own thread, and of 200."""
+    rng = np.random.default_rng(batch + chunk)
+    k_lens = [int(x) for x in rng.choice([1, 300, 8192, 8193, 51200], batch)]
+    q_lens = [1] * batch
+    if chunk:
+        for at, n in ((0, chunk), (batch - 1, 700)):
+            q_lens[at], k_lens[at] = n, n + int(rng.integers(0, 3000))
+    _check(f"small planner {batch} {chunk}", q_lens, k_lens, device=device)
+    _check(f"small planner {batch} {chunk} window", q_lens, k_lens, window=(9000, 0), device=device)
