@@ -256,6 +256,9 @@ constexpr int kLtThreads = 64 * kLtWaves;
 constexpr int kLtVocab = 16 * kLtVT * kLtWaves;  // vocab rows per workgroup: 640
 constexpr int kLtTileBytes = 16 * 64;            // a 16-row tile of a chunk
 
+// s_waitcnt immediate for lgkmcnt(0), expcnt unconstrained; the low bits hold vmcnt (below 16).
+constexpr unsigned kLtWait = 0x0070;
+
 template <int NT>
 struct LtBuf {
   unsigned char w[kLtWaves * kLtVT * kLtTileBytes];
@@ -312,10 +315,10 @@ __global__ __launch_bounds__(kLtThreads, 2) void logits_argmax_wide_kernel(
   auto step = [&](int c, const LtBuf<NT>& cur, LtBuf<NT>& next, bool steady) __attribute__((always_inline)) {
     // Chunk c has landed for this wave (chunk c + 1's loads may be out); after the barrier
     // for all, and all are done with chunk c - 1, whose buffer chunk c + 2 fills.
-    if (steady || c + 1 < chunks) __builtin_amdgcn_s_waitcnt(hx::kWaitVm0 | (kLtVT + XL));
-    else __builtin_amdgcn_s_waitcnt(hx::kWaitVm0);
+    // This wave's reads of chunk c - 1 have returned as well (lgkmcnt 0).
+    if (steady || c + 1 < chunks) __builtin_amdgcn_s_waitcnt(kLtWait | (kLtVT + XL));
+    else __builtin_amdgcn_s_waitcnt(kLtWait);
     // A plain barrier between compiler fences: __syncthreads would wait for chunk c + 1 too.
-    // This wave's reads of chunk c - 1 have returned, since its MFMAs used them.
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");

@@ -2275,7 +2275,6 @@ __device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws,
   const int urow = unit_ok ? u / it.hcount : 0;
   const int qh = g * ws.group + it.h0 + (unit_ok ? u - urow * it.hcount : 0);
   const int qpos = it.L - it.n + it.row0 + urow;
-  const bool busy = u0 < units;  // wave-uniform
 
   // Q^T as the MFMA B operand: lane holds its unit's dims 32st + 8(lane>>4)..+7.
   uint4 qf[NS];
@@ -2357,7 +2356,9 @@ __device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws,
     for (int j = 0; j < NP; ++j) *reinterpret_cast<uint4*>(lds.tile.v + v_at[j]) = vreg[j];
     __syncthreads();
     if (t + 1 < t_end) load_tile(t + 1);
-    if (!busy) continue;
+    // Tiles none of the wave's units sees (past a causal edge, or no units) are left out.
+    const int own = t * kTile + (DEC ? 16 * w : 0);  // the wave's keys: own .. own + 16 NB - 1
+    if (!__any(klo <= own + 16 * NB - 1 && khi >= own)) continue;
 
     // S^T: lane holds keys 16kb + 4(lane>>4) + i of unit lane & 15 (decode: kb is the wave).
     hx::f32x4_t s[NB];
@@ -2371,7 +2372,7 @@ __device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws,
         const uint4 kf = *reinterpret_cast<const uint4*>(lds.tile.k + kr * WideLds<DP>::kKRow + 16 * (4 * st + gg));
         s[kb] = E::mfma16x16x32(hx::as_v8<T>(kf), hx::as_v8<T>(qf[st]), s[kb]);
       }
-    const int key_base = t * kTile + (DEC ? 16 * w : 0) + 4 * gg;  // of s[0][0]
+    const int key_base = own + 4 * gg;  // of s[0][0]
     // Masked only where some lane's keys are not all visible (a wave-uniform test).
     if (__any(key_base < klo || key_base + 16 * (NB - 1) + 3 > khi)) {
 #pragma unroll

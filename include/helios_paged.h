@@ -390,7 +390,8 @@ size_t hx_varlen_attn_error_word_offset(void);
  * GPU it runs on until the process ends. The call allocates nothing: the array's device
  * address is looked up once per GPU, at that GPU's first call (make that first call
  * outside graph capture), with the stream's GPU current.
- *   - A shape whose workspace (hx_varlen_attn_workspace_bytes) exceeds the array
+ *   - A shape whose workspace (hx_varlen_attn_workspace_bytes; for shapes served by the
+ *     any-head_dim kernel, that of the same heads at head_dim 128) exceeds the array
  *     returns HX_E_TOO_LARGE before any launch. Decode ticks of up to ~15000 256-key
  *     splits fit, and so do the mixed and long-context ticks of the Qwen3-4B
  *     workloads (about 71-100 MiB).
