@@ -10,8 +10,8 @@
 //
 // All three are HBM / L2 streams with little arithmetic: 16-byte accesses, one workgroup per
 // row for the norm (a row stays in registers between its statistics and its output). At
-// 1152 rows of 2560 and ffn 9728 a norm takes 6.6 us (23.6 MB, 3.6 TB/s, of which about 2 us
-// are launch and one row's chain) and SwiGLU 13.1 us (67 MB, 5.1 TB/s): 26 us a layer. The op
+// 1152 rows of 2560 and ffn 9728 a norm takes 6.6 us (23.6 MB, 3.6 TB/s)
+// and SwiGLU 13.1 us (67 MB, 5.1 TB/s): 26 us a layer. The op
 // sequence's elementwise launches took 137 us a layer.
 
 #include "hx_common.h"

@@ -244,8 +244,9 @@ __global__ __launch_bounds__(kLgThreads) void logits_argmax_kernel(
 // The same product for many logit rows, where reading fragments from LDS costs more than the
 // weight stream: 8 waves x 5 MFMA tiles of vocab rows, so that an x fragment read feeds five
 // MFMAs instead of two, in one workgroup per CU (HBM and MFMA bound in turn: 129 rows take
-// 177 us, 4.4 TB/s of weights and 0.63 PFLOP/s; 64 rows and fewer are faster above). Weights and x go from memory straight into
-// LDS, 32 hidden elements at a time, into three buffers used in turn: two chunks are in
+// 177 us, 4.4 TB/s of weights; 64 rows and fewer are faster above). The first pass over a
+// table not read before loses 7 us at 129 rows (250 us against 243), a repeated one gains
+// 15. Weights and x go from memory straight into LDS, 32 hidden elements at a time, into three buffers used in turn: two chunks are in
 // flight while one is consumed, and a chunk costs one wait and one barrier.
 //
 // LDS rows are 64 bytes; the 16-byte piece at position p of row r is piece p ^ ((r >> 2) & 3),
