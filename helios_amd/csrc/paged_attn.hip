@@ -2254,10 +2254,175 @@ struct WideLds {
     __attribute__((aligned(16))) float o[4][kWideDecUnits][DP];  // the waves' results of a decode item
   };
   float m[4][kWideDecUnits], l[4][kWideDecUnits];
+  int odd[4];  // per wave: whether a sum of its is infinite or NaN
 };
 
+// The bits of a value that may be a NaN. The build assumes that no operand of a comparison is
+// one, and turns comparisons of a float's bits into those of the float; behind an empty asm
+// the compiler does not know that these are one's.
+__device__ __forceinline__ uint32_t raw_bits(float x) {
+  uint32_t b = __float_as_uint(x);
+  asm("" : "+v"(b));
+  return b;
+}
+__device__ __forceinline__ bool is_inf(float x) { return (raw_bits(x) & 0x7fffffffu) == 0x7f800000u; }
+__device__ __forceinline__ bool is_finite(float x) { return (raw_bits(x) & 0x7fffffffu) < 0x7f800000u; }
+
+// x + w * y for partial results. With ODD an infinite y counts however small its weight: the
+// sum over the whole row would have it so.
+template <bool ODD>
+__device__ __forceinline__ float add_weighed(float w, float y, float x) {
+  return ODD && is_inf(y) ? x + y : fmaf(w, y, x);
+}
+
+// Result (acc / l, four dims from d0) of one unit: output row piece, or partial.
+template <typename T>
+__device__ __forceinline__ void wide_store(const RunArgs& a, const WideShape& ws, const WideItem& it, int row, int head,
+                                           int d0, float ml, float ll, const float (&x)[4]) {
+  if (it.splits > 1) {
+    const int64_t slot = it.slot0 + (int64_t)row * it.splits;
+    if (slot >= a.slot_cap) return;
+    float* const part_o = reinterpret_cast<float*>(a.part_o);
+    *reinterpret_cast<float4*>(part_o + (slot * a.hq + head) * ws.head_dim + d0) = make_float4(x[0], x[1], x[2], x[3]);
+    if (d0 == 0) a.part_ml[slot * a.hq + head] = make_float2(ml, ll);
+    return;
+  }
+  const float inv = ll > 0.f ? 1.f / ll : 0.f;
+  const int64_t orow = it.q0 + it.row0 + row;
+  *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + orow * a.o_row + (int64_t)head * a.o_head + d0) =
+      make_uint2(hx::pack2_round<T>(x[0] * inv, x[1] * inv), hx::pack2_round<T>(x[2] * inv, x[3] * inv));
+  if (a.lse && d0 == 0)
+    a.lse[(int64_t)head * a.total_q + orow] = ll > 0.f ? (ml + (log2f(ll) - wide_p_shift<T>())) * kLn2 : -INFINITY;
+}
+
+// The waves' results of a decode item, from LDS, merged and stored. ODD: some are infinite or NaN.
+template <typename T, int DP, bool ODD>
+__device__ __forceinline__ void wide_merge_waves(const RunArgs& a, const WideShape& ws, const WideLds<DP>& lds,
+                                                 const int g, const WideItem& it) {
+  const int quads = ws.head_dim / 4;
+  for (int i = hx::tid_x(); i < it.hcount * quads; i += kWideThreads) {
+    const int h = i / quads, d0 = 4 * (i - h * quads);
+    float mm = -INFINITY, ll = 0.f, x[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ww = 0; ww < 4; ++ww) mm = fmaxf(mm, lds.m[ww][h]);
+#pragma unroll
+    for (int ww = 0; ww < 4; ++ww) {
+      const float mw = lds.m[ww][h];
+      const float alpha = mw == -INFINITY ? 0.f : hx::fast_exp2(mw - mm);
+      const float4 o4 = *reinterpret_cast<const float4*>(&lds.o[ww][h][d0]);
+      ll = fmaf(alpha, lds.l[ww][h], ll);
+      x[0] = add_weighed<ODD>(alpha, o4.x, x[0]);
+      x[1] = add_weighed<ODD>(alpha, o4.y, x[1]);
+      x[2] = add_weighed<ODD>(alpha, o4.z, x[2]);
+      x[3] = add_weighed<ODD>(alpha, o4.w, x[3]);
+    }
+    wide_store<T>(a, ws, it, 0, g * ws.group + it.h0 + h, d0, mm, ll, x);
+  }
+}
+
+// An item key by key on the VALU, for V with infinite or NaN elements. In P V as matrix
+// products such an element spoils more than the rows that see it: 0 * inf is NaN, for a key
+// that the mask hides as for a remainder operand of P that is 0, and remainders have either
+// sign. The kernel comes here when wide_item reports an infinite or NaN sum. Four lanes share
+// a unit (16-byte pieces r, r + 4, ... of the head dim); a decode item's waves take every
+// fourth key.
+template <typename T, int DP>
+__device__ __forceinline__ void wide_odd_item(const RunArgs& a, const WideShape& ws, WideLds<DP>& lds, const int g,
+                                              const WideItem& it, const bool decode) {
+  typedef hx::Elem<T> E;
+  constexpr int NC = DP / 32;  // pieces per lane
+  int tid = hx::tid_x();
+  asm volatile("" : "+v"(tid));  // nothing derived from it is computed ahead, in registers
+  const int lane = tid & 63, r = lane & 3;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int D = ws.head_dim;
+  const int u = (decode ? 0 : 16 * w) + (lane >> 2);
+  const bool unit_ok = u < it.rows * it.hcount;
+  const int urow = unit_ok ? u / it.hcount : 0;
+  const int qh = g * ws.group + it.h0 + (unit_ok ? u - urow * it.hcount : 0);
+  const int qpos = it.L - it.n + it.row0 + urow;
+  int klo = it.k_begin, khi = unit_ok ? it.k_end - 1 : -1;
+  if (a.win_left >= 0) klo = max(klo, qpos - a.win_left);
+  if (a.win_right >= 0) khi = min(khi, qpos + a.win_right);
+
+  const T* const qp = reinterpret_cast<const T*>(a.q) + query_row(a, it.q0 + it.row0 + urow) * a.q_row +
+                      (int64_t)qh * a.q_head;
+  float o[NC][8], m = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[j][e] = 0.f;
+#pragma unroll 1
+  for (int t0 = it.k_begin / kTile * kTile; t0 < it.k_end; t0 += kTile) {
+    int64_t row = (int64_t)it.kvb + t0;
+    if (a.page_size > 0) {
+      const int pg = t0 / a.page_size;
+      const int page = a.bt[(int64_t)it.b * a.bt_stride + pg];
+      // A bad id has set the error word by now.
+      row = ((unsigned)page < (unsigned)a.num_pages ? (int64_t)page * a.page_size : 0) + (t0 - pg * a.page_size);
+    }
+    const int keys = min(it.k_end - t0, kTile);
+#pragma unroll 1
+    for (int kk = decode ? w : 0; kk < keys; kk += decode ? 4 : 1) {
+      const int key = t0 + kk;
+      const bool seen = key >= klo && key <= khi;  // the same for a unit's four lanes
+      if (!__any(seen)) continue;
+      const int64_t at = (row + kk) * a.kv_row + (int64_t)g * a.kv_head;
+      float s = 0.f;
+#pragma unroll 1
+      for (int d = 8 * r; d < D; d += 32) {
+        const uint4 k4 = ld16(reinterpret_cast<const T*>(a.k) + at + d), q4 = ld16(qp + d);
+        const uint32_t kw[4] = {k4.x, k4.y, k4.z, k4.w}, qw[4] = {q4.x, q4.y, q4.z, q4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = fmaf(E::hi(qw[e]), E::hi(kw[e]), fmaf(E::lo(qw[e]), E::lo(kw[e]), s));
+      }
+      s += __shfl_xor(s, 1);
+      s += __shfl_xor(s, 2);
+      s *= a.scale_log2;
+      const float mt = seen ? fmaxf(m, s) : m;
+      // A NaN score makes its row NaN (it is no maximum, also where it is the first).
+      const bool counts = seen && raw_bits(s) != 0xff800000u;
+      const float p = counts ? hx::fast_exp2(s + (wide_p_shift<T>() - (mt != -INFINITY ? mt : 0.f))) : 0.f;
+      const float alpha = m != -INFINITY ? hx::fast_exp2(m - mt) : 0.f;
+      m = mt;
+      l = fmaf(l, alpha, p);
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        const int d = 8 * (r + 4 * j);
+        if (d >= D) continue;
+        const uint4 v4 = ld16(reinterpret_cast<const T*>(a.v) + at + d);
+        const uint32_t vw[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          o[j][2 * e] = seen ? fmaf(p, E::lo(vw[e]), o[j][2 * e] * alpha) : o[j][2 * e];
+          o[j][2 * e + 1] = seen ? fmaf(p, E::hi(vw[e]), o[j][2 * e + 1] * alpha) : o[j][2 * e + 1];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const int d = 8 * (r + 4 * j);
+    if (!unit_ok || d >= D) continue;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float x[4] = {o[j][4 * h], o[j][4 * h + 1], o[j][4 * h + 2], o[j][4 * h + 3]};
+      if (decode) *reinterpret_cast<float4*>(&lds.o[w][u][d + 4 * h]) = make_float4(x[0], x[1], x[2], x[3]);
+      else wide_store<T>(a, ws, it, urow, qh, d + 4 * h, m, l, x);
+    }
+  }
+  if (!decode) return;
+  if (unit_ok && r == 0) {
+    lds.m[w][u] = m;
+    lds.l[w][u] = l;
+  }
+  __syncthreads();
+  wide_merge_waves<T, DP, true>(a, ws, lds, g, it);
+}
+
+// One item; true, and nothing stored, when one of its sums is infinite or NaN.
 template <typename T, int DP, bool DEC>
-__device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws, WideLds<DP>& lds, const int g,
+__device__ __forceinline__ bool wide_item(const RunArgs& a, const WideShape& ws, WideLds<DP>& lds, const int g,
                                           const WideItem& it) {
   typedef hx::Elem<T> E;
   constexpr int kPieces = DP / 8;                       // 16-byte pieces of a padded row
@@ -2438,22 +2603,17 @@ __device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws,
   if (bad_page && tid == 0) atomicOr(&a.hdr[H_ERR], HX_WERR_BAD_PAGE);
   l = hx::add_xor32(hx::add_xor16(l));
 
-  float* const part_o = reinterpret_cast<float*>(a.part_o);
-  // Result (acc / l, four dims from d0) of one unit: output row piece, or partial.
-  auto store = [&](int row, int head, int d0, float ml, float ll, const float (&x)[4]) {
-    if (it.splits > 1) {
-      const int64_t slot = it.slot0 + (int64_t)row * it.splits;
-      if (slot >= a.slot_cap) return;
-      *reinterpret_cast<float4*>(part_o + (slot * a.hq + head) * D + d0) = make_float4(x[0], x[1], x[2], x[3]);
-      if (d0 == 0) a.part_ml[slot * a.hq + head] = make_float2(ml, ll);
-      return;
-    }
-    const float inv = ll > 0.f ? 1.f / ll : 0.f;
-    const int64_t orow = it.q0 + it.row0 + row;
-    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(a.out) + orow * a.o_row + (int64_t)head * a.o_head + d0) =
-        make_uint2(hx::pack2_round<T>(x[0] * inv, x[1] * inv), hx::pack2_round<T>(x[2] * inv, x[3] * inv));
-    if (a.lse && d0 == 0)
-      a.lse[(int64_t)head * a.total_q + orow] = ll > 0.f ? (ml + (log2f(ll) - wide_p_shift<T>())) * kLn2 : -INFINITY;
+  // Whether a sum of this item, in any wave, is infinite or NaN.
+  auto vote = [&]() {
+    uint32_t top = 0;
+#pragma unroll
+    for (int db = 0; db < NO; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) top = max(top, raw_bits(oacc[db][i]) & 0x7fffffffu);
+    const int odd = __any(top >= 0x7f800000u);
+    if (lane == 0) lds.odd[w] = odd;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(lds.odd[0] | lds.odd[1] | lds.odd[2] | lds.odd[3]) != 0;
   };
   if constexpr (DEC) {
     __syncthreads();  // the last tile's readers are done
@@ -2465,34 +2625,19 @@ __device__ __forceinline__ void wide_item(const RunArgs& a, const WideShape& ws,
     for (int db = 0; db < NO; ++db)
       *reinterpret_cast<float4*>(&lds.o[w][lane & 15][16 * db + 4 * gg]) =
           make_float4(oacc[db][0], oacc[db][1], oacc[db][2], oacc[db][3]);
-    __syncthreads();
-    const int quads = D / 4;
-    for (int i = tid; i < it.hcount * quads; i += kWideThreads) {
-      const int h = i / quads, d0 = 4 * (i - h * quads);
-      float mm = -INFINITY, ll = 0.f, x[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ww = 0; ww < 4; ++ww) mm = fmaxf(mm, lds.m[ww][h]);
-#pragma unroll
-      for (int ww = 0; ww < 4; ++ww) {
-        const float mw = lds.m[ww][h];
-        const float alpha = mw == -INFINITY ? 0.f : hx::fast_exp2(mw - mm);
-        const float4 o4 = *reinterpret_cast<const float4*>(&lds.o[ww][h][d0]);
-        ll = fmaf(alpha, lds.l[ww][h], ll);
-        x[0] = fmaf(alpha, o4.x, x[0]);
-        x[1] = fmaf(alpha, o4.y, x[1]);
-        x[2] = fmaf(alpha, o4.z, x[2]);
-        x[3] = fmaf(alpha, o4.w, x[3]);
-      }
-      store(0, g * ws.group + it.h0 + h, d0, mm, ll, x);
-    }
+    if (vote()) return true;
+    wide_merge_waves<T, DP, false>(a, ws, lds, g, it);
   } else {
+    // (An item without tiles has no sums, and no barrier since the last vote.)
+    if (t_begin < t_end && vote()) return true;
 #pragma unroll
     for (int db = 0; db < NO; ++db) {
       const int d0 = 16 * db + 4 * gg;
       const float x[4] = {oacc[db][0], oacc[db][1], oacc[db][2], oacc[db][3]};
-      if (unit_ok && d0 < D) store(urow, qh, d0, m, l, x);
+      if (unit_ok && d0 < D) wide_store<T>(a, ws, it, urow, qh, d0, m, l, x);
     }
   }
+  return false;
 }
 
 // A work-list entry, the same for the whole workgroup: kept in scalar registers.
@@ -2596,8 +2741,8 @@ __global__ __launch_bounds__(kWideThreads, DP <= 64 ? 4 : DP == 128 ? 3 : 2) voi
     it.h0 = hb * per;
     it.hcount = min(per, ws.group - it.h0);
     if (it.hcount < 1) continue;
-    if (decode) wide_item<T, DP, true>(a, ws, lds, g, it);
-    else wide_item<T, DP, false>(a, ws, lds, g, it);
+    const bool odd = decode ? wide_item<T, DP, true>(a, ws, lds, g, it) : wide_item<T, DP, false>(a, ws, lds, g, it);
+    if (odd) wide_odd_item<T, DP>(a, ws, lds, g, it, decode);
   }
 }
 
@@ -2654,6 +2799,18 @@ __global__ __launch_bounds__(kWideThreads) void wide_combine_kernel(RunArgs a, W
           x[3] = fmaf(wt, o4[j].w, x[3]);
         }
         m = mn;
+      }
+      if (!(is_finite(x[0]) && is_finite(x[1]) && is_finite(x[2]) && is_finite(x[3]))) {
+        x[0] = x[1] = x[2] = x[3] = 0.f;
+        for (int sp = 0; sp < splits; ++sp) {
+          const float ms = a.part_ml[base + (int64_t)sp * a.hq].x;
+          const float wt = ms != -INFINITY ? hx::fast_exp2(ms - m) : 0.f;
+          const float4 o4 = *reinterpret_cast<const float4*>(part_o + (base + (int64_t)sp * a.hq) * D + d0);
+          x[0] = add_weighed<true>(wt, o4.x, x[0]);
+          x[1] = add_weighed<true>(wt, o4.y, x[1]);
+          x[2] = add_weighed<true>(wt, o4.z, x[2]);
+          x[3] = add_weighed<true>(wt, o4.w, x[3]);
+        }
       }
       const float inv = l > 0.f ? 1.f / l : 0.f;
       const int64_t orow = c.w + r;

@@ -93,3 +93,84 @@ def test_wide_expanded_packed_keys(device):
     want = v[0].repeat_interleave(3, dim=0).expand(5, 6, 64)
     # equal weights of one row: the row itself, up to the rounding of fp32 sums
     assert torch.equal(out, want)
+
+
+def _plant(tick, seed):
+    """Infinities and NaNs for V: {sequence: {(key, kv head, dim): value}}."""
+    rng = np.random.default_rng(seed)
+    w, planted = tick.w, {}
+    hkv, d = w.n_kv_heads, w.head_dim
+    for b in (2, 6, len(w.k_lens) - 1):  # decode rows of one and of five splits, the last chunk
+        L, at = w.k_lens[b], {}
+        for g in range(hkv):
+            at[(int(rng.integers(0, L)), g, 0)] = np.inf
+            at[(L - 1, g, 1)] = -np.inf
+            at[(int(rng.integers(0, L)), g, 2)] = np.inf
+            at[(L - 2, g, 2)] = np.inf
+            at[(0, g, 3)] = np.inf
+            at[(L // 2, g, 3)] = -np.inf
+            at[(L // 3, g, 4)] = np.nan
+            at[(L - 1, g, d - 1)] = np.inf
+        planted[b] = at
+    return planted
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", [(16, 4, 64), (3, 1, 8), (6, 2, 72), (34, 2, 96), (6, 1, 128), (4, 1, 256)])
+def test_infinite_and_nan_values(device, hq, hkv, d, dtype):
+    """An infinite element of V gives +-inf to the rows that see its key, NaN where both signs
+    or a NaN are seen, and nothing to the others, whose results stay what they were; a NaN in K
+    makes the rows that see it NaN. Key 0 is drawn to the queries, so that p is 1 there in many
+    rows, exact in either type; the last keys are masked for the chunk's earlier rows."""
+    say("wide inf", hq, hkv, d, dtype)
+    tick = _tick(Q_LENS, K_LENS, hq, hkv, d, dtype, device, 700 + d)
+    w = tick.w
+    k_flat, v_flat = tick.k_pool.view(-1, hkv, d), tick.v_pool.view(-1, hkv, d)
+    at = lambda b, key: w.tables[b][key // 256] * 256 + key % 256  # noqa: E731
+    for b in range(w.batch):
+        rows = tick.q[w.cu_seq_q[b]:w.cu_seq_q[b + 1]].float().view(-1, hkv, hq // hkv, d).mean((0, 2))
+        k_flat[at(b, 0)] = (rows / rows.norm(dim=-1, keepdim=True) * 4 * d ** 0.5).to(dtype)
+    for window in ((-1, 0), (100, 5)):
+        before, lse0 = tick.attend(window=window, exact_grid=True, return_lse=True)
+        planted = _plant(tick, d)
+        keep = v_flat.clone()
+        for b, elements in planted.items():
+            for (key, g, dim), value in elements.items():
+                v_flat[at(b, key), g, dim] = value
+        k_keep, nan_keys = k_flat.clone(), {4: 0, 5: 512, 11: 256}
+        for b, key in nan_keys.items():
+            k_flat[at(b, key), hkv - 1, 0] = np.nan
+        out, lse = tick.attend(window=window, exact_grid=True, return_lse=True)
+        want = before.double().cpu().numpy()
+        touched = np.zeros(want.shape, bool)
+        for b, elements in planted.items():
+            n, L = w.q_lens[b], w.k_lens[b]
+            for i in range(n):
+                pos = L - n + i
+                lo = 0 if window[0] < 0 else max(0, pos - window[0])
+                hi = min(L - 1, pos + window[1])
+                for (key, g, dim), value in elements.items():
+                    if lo <= key <= hi:
+                        heads = slice(g * (hq // hkv), (g + 1) * (hq // hkv))
+                        row = w.cu_seq_q[b] + i
+                        with np.errstate(invalid="ignore"):
+                            want[row, heads, dim] = value if not touched[row, heads.start, dim] else \
+                                want[row, heads, dim] + value
+                        touched[row, heads, dim] = True
+        for b, key in nan_keys.items():
+            for i in range(w.q_lens[b]):
+                pos = w.k_lens[b] - w.q_lens[b] + i
+                if (0 if window[0] < 0 else pos - window[0]) <= key <= pos + window[1]:
+                    want[w.cu_seq_q[b] + i, hq - hq // hkv:] = np.nan
+                    touched[w.cu_seq_q[b] + i, hq - hq // hkv:] = True
+        got = out.double().cpu().numpy()
+        assert touched.any() and not np.isfinite(want[touched]).any()
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        np.testing.assert_array_equal(got[touched & ~np.isnan(want)], want[touched & ~np.isnan(want)])
+        # the rest: fp32 sums in another order, one rounding step apart at most
+        rest, ulp = ~touched, 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+        assert (np.abs(got[rest] - want[rest]) <= ulp * np.abs(want[rest]) + 1e-6).all()
+        same = ~touched.all(axis=-1).T  # the log-sum-exp of a NaN row is not specified
+        assert np.abs(lse.cpu().numpy() - lse0.cpu().numpy())[same].max() < 1e-4
+        v_flat.copy_(keep)
+        k_flat.copy_(k_keep)
