@@ -2179,9 +2179,13 @@ __global__ __launch_bounds__(kChunkThreads, 2) void chunk_pair_kernel(RunArgs a0
 // their key tiles like the tuned kernels' when they would not fill the GPU. The launch is
 // persistent (kWideWGs workgroups walk the lists), since the item counts are known on the
 // device only.
-// P keeps fp32's accuracy: it goes into P V as two MFMA operands, its rounding to the
-// element type and the remainder (17 bits or more of p), and the splits' partial results
-// stay in fp32. q . k is exact products in fp32 sums.
+// P stays in fp32: it goes into P V as its roundings to the element type, each of what the
+// ones before left. Three bf16 hold all 24 bits; two fp16 hold 23 of a p above 2^-13, which is
+// below the error of the exp, and 2^-37 absolute of a smaller one (p is scaled by 2^12). Two
+// bf16 (17 bits) showed where values cancel: 100 keys against 100 with weights 1/2000 apart
+// came out 0.57 % off instead of 0.18 %, of which the output's rounding is 0.17 %. The third
+// costs chunks 5-13 % and decode rows, whose 16 keys fill half an operand, nothing. The splits'
+// partial results stay in fp32. q . k is exact products in fp32 sums.
 // Bound by latency at these sizes. 24 decode rows of 200-2048 keys and chunks of 512 and
 // 333 rows, 16/4 heads, d = 64: 18.6 us and 4.8 us for the merge; scores and P V on the VALU,
 // 16 units a workgroup and no splits, took 284 us. Two tiles in flight instead of one gained
@@ -2430,6 +2434,8 @@ __device__ __forceinline__ bool wide_item(const RunArgs& a, const WideShape& ws,
   constexpr int NS = DP / 32, NO = DP / 16;             // QK^T steps, O blocks
   constexpr int NB = DEC ? 1 : 4;                       // 16-key blocks of a tile a wave takes
   constexpr int NK = DEC ? 1 : 2;                       // P V key steps per tile
+  constexpr int kPParts = std::is_same<T, _Float16>::value ? 2 : 3;  // P's roundings to the type, see above
+  constexpr int kPOps = DEC ? (kPParts + 1) / 2 : kPParts;           // and the operands they fill
   const int tid = hx::tid_x(), lane = tid & 63, gg = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int D = ws.head_dim;
@@ -2562,7 +2568,6 @@ __device__ __forceinline__ bool wide_item(const RunArgs& a, const WideShape& ws,
       m = mt;
     }
     const float neg_m = m == -INFINITY ? 0.f : wide_p_shift<T>() - m;
-    uint4 ph[NK], pl[NK];
 #pragma unroll
     for (int kb = 0; kb < NB; ++kb) {
 #pragma unroll
@@ -2571,32 +2576,37 @@ __device__ __forceinline__ bool wide_item(const RunArgs& a, const WideShape& ws,
         l += s[kb][i];
       }
     }
-#pragma unroll
-    for (int ks = 0; ks < NK; ++ks) {
-      uint32_t hi[4] = {0u, 0u, 0u, 0u}, lo[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int j = 0; j < (DEC ? 2 : 4); ++j) {
-        const float x = s[DEC ? 0 : 2 * ks + (j >> 1)][2 * (j & 1)], y = s[DEC ? 0 : 2 * ks + (j >> 1)][2 * (j & 1) + 1];
-        hi[j] = hx::pack2_round<T>(x, y);
-        lo[j] = hx::pack2_round<T>(x - E::lo(hi[j]), y - E::hi(hi[j]));
-      }
-      ph[ks] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-      pl[ks] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-    }
     // V^T operands, read transposed: keys {r0 + 0..3, r0 + 16 + 0..3} of dim 16db + j per
-    // lane (chunk_body's read_v); a decode wave's 16 keys fill the first half only.
+    // lane (chunk_body's read_v). A decode wave's 16 keys fill half an operand: V twice, and
+    // two parts of P side by side.
     const int i16 = lane & 15;
 #pragma unroll
     for (int ks = 0; ks < NK; ++ks) {
+      uint32_t part[4][4] = {};
+#pragma unroll
+      for (int j = 0; j < (DEC ? 2 : 4); ++j) {
+        float x = s[DEC ? 0 : 2 * ks + (j >> 1)][2 * (j & 1)], y = s[DEC ? 0 : 2 * ks + (j >> 1)][2 * (j & 1) + 1];
+#pragma unroll
+        for (int n = 0; n < kPParts; ++n) {
+          part[n][j] = hx::pack2_round<T>(x, y);
+          x -= E::lo(part[n][j]);
+          y -= E::hi(part[n][j]);
+        }
+      }
+      uint4 pp[kPOps];
+#pragma unroll
+      for (int n = 0; n < kPOps; ++n)
+        pp[n] = DEC ? make_uint4(part[2 * n][0], part[2 * n][1], part[2 * n + 1][0], part[2 * n + 1][1])
+                    : make_uint4(part[n][0], part[n][1], part[n][2], part[n][3]);
       const int r0 = (DEC ? 16 * w : 32 * ks) + 4 * gg + (i16 >> 2);
       const uint8_t* vp = lds.tile.v + r0 * WideLds<DP>::kVRow + 8 * (i16 & 3);
 #pragma unroll
       for (int db = 0; db < NO; ++db) {
         const uint2 lo = hx::ld8_lds_tr16(vp + 32 * db);
-        const uint2 hi = DEC ? make_uint2(0u, 0u) : hx::ld8_lds_tr16(vp + 16 * WideLds<DP>::kVRow + 32 * db);
+        const uint2 hi = DEC ? lo : hx::ld8_lds_tr16(vp + 16 * WideLds<DP>::kVRow + 32 * db);
         const uint4 vf = make_uint4(lo.x, lo.y, hi.x, hi.y);
-        oacc[db] = E::mfma16x16x32(hx::as_v8<T>(vf), hx::as_v8<T>(ph[ks]), oacc[db]);
-        oacc[db] = E::mfma16x16x32(hx::as_v8<T>(vf), hx::as_v8<T>(pl[ks]), oacc[db]);
+#pragma unroll
+        for (int n = 0; n < kPOps; ++n) oacc[db] = E::mfma16x16x32(hx::as_v8<T>(vf), hx::as_v8<T>(pp[n]), oacc[db]);
       }
     }
   }

@@ -133,8 +133,8 @@ int hx_kv_gather(const void* pool, int32_t num_pool_pages, int32_t page_size,
  * query heads share each K/V read, and a deterministic combine; chunk rows (n_b > 1)
  * run a bf16/fp16 MFMA kernel. Every other shape runs one MFMA kernel for all rows over
  * the same kind of splits, blocks of 64 (row, query head) pairs of a KV head sharing each
- * 64-key K/V tile through LDS, with fp32 scores, P to 17 bits and fp32 partials, and a
- * deterministic combine. In a workspace below the size stated here but not below that of
+ * 64-key K/V tile through LDS, with fp32 scores, P and partials, and a deterministic
+ * combine. In a workspace below the size stated here but not below that of
  * the same heads at head_dim 128, it runs without splits.
  *
  * The workspace (size from hx_varlen_attn_workspace_bytes, 256-byte aligned) holds

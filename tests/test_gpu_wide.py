@@ -41,17 +41,44 @@ def test_wide_edges(device, hq, hkv, d, dtype):
         assert np.abs(lse.cpu().numpy() - ref_lse).max() < 1e-4
 
 
-def test_wide_keeps_p_in_more_than_16_bits(device):
-    """With V near 1 every output is a sum of many p times nearly the same value: rounding p
-    to bf16 before the product, with l summed unrounded, would show as 2^-9 of the output
-    with random sign; the output's own rounding is bounded by half its spacing."""
+def test_wide_constant_values(device):
+    """Constant V: the weights of a row sum to one, so each output rounds to that value."""
     tick = _tick([1, 40], [1500, 700], 8, 2, 64, torch.bfloat16, device, 41)
     tick.v_pool.fill_(1.0)
     tick.v_pool[..., ::2] = 0.75
     out = tick.attend()
     torch.cuda.synchronize()
-    # exact weights of one sum to 1: both values are representable, so the result rounds to them
     assert (out[..., 1::2] == 1.0).all() and (out[..., ::2] == 0.75).all()
+
+
+@pytest.mark.parametrize("rows", [1, 20])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wide_keeps_p_in_fp32(device, dtype, rows):
+    """A hundred keys of weight p1 with V = 1 against a hundred of p2 with V = -1 and one key
+    of weight 1 with V = 0. Scores come from one dim, so they are exact; p1 - p2 is at least
+    2.4e-4. In fp32 the two exps (2^-23 each) move the output by 1e-3 of itself, and so do 400
+    roundings of sums up to 1 (2^-24 each, of a sum of 0.024); the rounding of the output adds
+    half a step. Emulated errors with P in one, two and three operands: bf16 3.4, 5.7e-3 and
+    1.8e-3; fp16 1.0, 4.4e-4 and 4.4e-4."""
+    say("wide p", dtype, rows)
+    hq, n, d = 16, 100, 64
+    a = torch.linspace(0.5, 3.5, hq).to(dtype)
+    q = torch.zeros(rows, hq, d, dtype=dtype, device=device)
+    q[:, :, 0] = a.to(device)
+    # masked keys fill up to a causal chunk: every row sees the first 2 n + 1
+    k = torch.zeros(2 * n + 1 + rows - 1, 1, d, dtype=dtype, device=device)
+    v = torch.zeros_like(k)
+    k[1:2 * n + 1:2, :, 0], k[2:2 * n + 1:2, :, 0] = -0.5 - 2.0 ** -8, -0.5
+    v[1:2 * n + 1:2], v[2:2 * n + 1:2] = 1.0, -1.0
+    k[2 * n + 1:, :, 0] = -448.0  # of no weight
+    cu_q = torch.tensor([0, rows], dtype=torch.int32, device=device)
+    cu_k = torch.tensor([0, k.shape[0]], dtype=torch.int32, device=device)
+    out = ops.varlen_attn(q, k, v, cu_q, cu_k, rows, k.shape[0], is_causal=True, enable_gqa=True).double().cpu()
+    p1, p2 = (torch.exp(a.double() * b / 8) for b in (-0.5 - 2.0 ** -8, -0.5))
+    want = (n * (p1 - p2) / (1 + n * (p1 + p2))).view(1, hq, 1)
+    off = (out / want - 1).abs().max().item()
+    say("relative error", off)
+    assert off <= 2e-3 + (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -11)
 
 
 @pytest.mark.parametrize("hq,hkv,d", [(4, 1, 256), (8, 1, 136)])
