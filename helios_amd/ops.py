@@ -403,14 +403,16 @@ def block_linear(x: torch.Tensor, weight: torch.Tensor, *, norm_weight: torch.Te
         if tuple(norm_weight.shape) != (k,) or norm_weight.device != device or not norm_weight.is_floating_point():
             raise ValueError("norm_weight must be floating-point [K].")
         norm_weight = norm_weight.float().contiguous()  # no copy for the usual float32 vector
+    if k == 0:  # sums of no terms
+        zero = torch.zeros(shape, dtype=x.dtype, device=device)
+        return zero if residual is None else residual + zero
     out = torch.empty(shape, dtype=x.dtype, device=device)
-    if k:
-        code = _capi.lib().hx_skinny_gemm(
-            x.data_ptr(), k, x.numel() // k, weight.data_ptr(), k, cols, k, dtype,
-            None if norm_weight is None else norm_weight.data_ptr(), eps,
-            None if residual is None else residual.data_ptr(), cols, 1 if swiglu else 0,
-            out.data_ptr(), cols, _stream_ptr(device))
-        _capi.check(code, "hx_skinny_gemm")
+    code = _capi.lib().hx_skinny_gemm(
+        x.data_ptr(), k, x.numel() // k, weight.data_ptr(), k, cols, k, dtype,
+        None if norm_weight is None else norm_weight.data_ptr(), eps,
+        None if residual is None else residual.data_ptr(), cols, 1 if swiglu else 0,
+        out.data_ptr(), cols, _stream_ptr(device))
+    _capi.check(code, "hx_skinny_gemm")
     return out
 
 

@@ -116,6 +116,21 @@ def test_block_linear(device, rows, cols, k, dtype):
             assert (got - ref).abs().mean() <= 0.1 * ULP[dtype]
 
 
+def test_block_linear_of_no_terms(device):
+    """K = 0: the product is 0, whatever the output's memory held."""
+    say("block_linear K = 0")
+    x, w = (torch.empty(n, 0, dtype=torch.bfloat16, device=device) for n in (3, 4096))
+    norm = torch.empty(0, device=device)
+    residual = torch.randn(3, 4096, device=device).to(torch.bfloat16)
+    for n in (None, norm):
+        for kw, want in ((dict(), torch.zeros_like(residual)), (dict(residual=residual), residual),
+                         (dict(swiglu=True), torch.zeros_like(residual[:, :2048]))):
+            stale = torch.full_like(want, 7.0)
+            del stale  # the next allocation of this size
+            got = ops.block_linear(x, w, norm_weight=n, eps=1e-6, **kw)
+            assert torch.equal(got, want)
+
+
 def test_block_linear_refuses_other_shapes(device):
     x = torch.zeros(17, 64, dtype=torch.bfloat16, device=device)
     w = torch.zeros(32, 64, dtype=torch.bfloat16, device=device)
