@@ -144,7 +144,9 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(SkinnyArgs a) {
 #pragma unroll
   for (int v = 0; v < NV; ++v) acc[v] = hx::f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  // One wave's LDS accesses complete in order, so its stage needs no barrier.
+  // Lanes read what other lanes of the wave stored. One wave's LDS accesses complete in order,
+  // so its stage needs no barrier; the wavefront fences (no instruction) hold the compiler to
+  // the order of stores, reads and the next batch's stores.
   uint8_t* const stage = smem + w * kWaveBytes;
   auto consume = [&](int i, int b) __attribute__((always_inline)) {
 #pragma unroll
@@ -154,6 +156,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(SkinnyArgs a) {
         *reinterpret_cast<uint4*>(stage + v * kSkTileBytes + 1024 * j + 16 * lane) = wb[i][v][j];
       *reinterpret_cast<uint4*>(stage + NV * kSkTileBytes + 1024 * j + 16 * lane) = xb[i][j];
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if (b + D < b_end) {  // wave-uniform
       load_x(i, b + D);
       load_w(i, b + D);
@@ -180,6 +183,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_gemm_kernel(SkinnyArgs a) {
         acc[v] = E::mfma16x16x32(hx::as_v8<T>(wf), hx::as_v8<T>(xv), acc[v]);
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   };
   for (int b = b_begin; b < b_end; b += D) {
 #pragma unroll
