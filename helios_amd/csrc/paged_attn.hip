@@ -588,8 +588,16 @@ constexpr int kPlanSortBlocks = 256;
 // and per-wave totals, and four waves get through them sooner than sixteen (64 decode rows
 // 5.6 -> 3.9 us; 14, 64 and 76 blocks 12.3 -> 9.4, 9.7 -> 7.7 and 13.3 -> 12.0 us; 126 blocks
 // would be slower).
+// The split-size search has to fit them as well, one size (of up to max_k / 64) a thread and
+// 32 blocks' counts each. Beyond, 1024 threads are sooner: 32/8 heads, 1024 rows at 32768 keys
+// 16.0 against 17.5 us, 2048 rows 14.0 against 17.1; 16/4 heads of 64, 1024 rows at 16384 keys
+// 14.4 against 17.6.
 constexpr int kPlanSmallThreads = 256;
 constexpr int kPlanSmallBlocks = 96;
+constexpr int kPlanSmallSearch = 32 * kPlanSmallThreads;  // split sizes x blocks
+// For this many blocks a thread's walk over all costs less than dealing them out, with its
+// barriers (64 rows at 32768 keys 15.9 -> 14.9 us).
+constexpr int kPlanFewBlocks = 8;
 constexpr int kPlanOwnItems = 32;  // decode items a row's own thread writes
 static_assert(kPlanSortBlocks <= kPlanSmallThreads, "a thread per sorted block");
 
@@ -715,14 +723,17 @@ __global__ __launch_bounds__(TH) void plan_kernel(PlanArgs a) {
       // Workgroups at split size st0 + j for every j <= ncand, the blocks dealt over as many
       // threads as there are per candidate (one thread walking all blocks took 0.08 us a
       // block); the smallest fitting candidate wins an LDS atomicMin.
-      const int parts = TH / (ncand + 1);
+      const int parts = n_blk <= kPlanFewBlocks ? 1 : TH / (ncand + 1);
       const int part = tid / (ncand + 1), j = tid - part * (ncand + 1);
-      if (tid <= ncand) cand_wgs[tid] = 0;
-      __syncthreads();
+      if (parts > 1) {
+        if (tid <= ncand) cand_wgs[tid] = 0;
+        __syncthreads();
+      }
       if (part < parts && part < n_blk) {
         int wg = 0;
         for (int i = part; i < n_blk; i += parts) wg += chunk_split_count(fb_tiles[i], st0 + j);
-        atomicAdd(&cand_wgs[j], wg);
+        if (parts > 1) atomicAdd(&cand_wgs[j], wg);
+        else cand_wgs[j] = wg;
       }
       __syncthreads();
       const int64_t w0 = (int64_t)cand_wgs[0] * a.head_quads * a.hkv;
@@ -859,6 +870,9 @@ __global__ __launch_bounds__(TH) void plan_kernel(PlanArgs a) {
   int* const blk_key = cand_wgs;                      // free after the split search
   int* const blk_items = cand_wgs + kPlanSortBlocks;
   int* const blk_first = cand_wgs + 2 * kPlanSortBlocks;  // first item of the block
+  auto items_before = [&](int key, int i, int j) {  // items of block j if it comes before block i
+    return blk_key[j] > key || (blk_key[j] == key && j < i) ? blk_items[j] : 0;
+  };
   if (by_length) {
     if (tid < n_blk) {
       const int S = chunk_split_count(fb_tiles[tid], split_tiles, keep_tiles);
@@ -866,19 +880,19 @@ __global__ __launch_bounds__(TH) void plan_kernel(PlanArgs a) {
       blk_items[tid] = S * a.head_quads;
     }
     __syncthreads();
-    // 16 threads rank each block (4 when there are many): items of the blocks before it.
+    // 16 threads rank each block (4 when there are many): items of the blocks before it. A few
+    // blocks are ranked by their own threads below, without another barrier.
     const int sh = n_blk <= TH / 16 ? 4 : 2;
-    for (int i = tid >> sh; i < n_blk; i += TH >> sh) {
-      const int key = blk_key[i];
-      int before = 0;
-      for (int j = tid & ((1 << sh) - 1); j < n_blk; j += 1 << sh) {
-        const int kj = blk_key[j];
-        before += kj > key || (kj == key && j < i) ? blk_items[j] : 0;
+    if (n_blk > kPlanFewBlocks) {
+      for (int i = tid >> sh; i < n_blk; i += TH >> sh) {
+        const int key = blk_key[i];
+        int before = 0;
+        for (int j = tid & ((1 << sh) - 1); j < n_blk; j += 1 << sh) before += items_before(key, i, j);
+        for (int m = 1; m < (1 << sh); m <<= 1) before += __shfl_xor(before, m);
+        if ((tid & ((1 << sh) - 1)) == 0) blk_first[i] = before;
       }
-      for (int m = 1; m < (1 << sh); m <<= 1) before += __shfl_xor(before, m);
-      if ((tid & ((1 << sh) - 1)) == 0) blk_first[i] = before;
+      __syncthreads();
     }
-    __syncthreads();
   }
   for (int i = tid; i < n_blk; i += TH) {
     int k, blk;
@@ -889,7 +903,12 @@ __global__ __launch_bounds__(TH) void plan_kernel(PlanArgs a) {
     const int S = chunk_split_count(fb_tiles[i], split_tiles, keep_tiles);
     const int rows = min(a.rows_per_item, n - row0);
     int item0 = cs_off_p[k] + fb_p[i] - fb_p[f0];
-    if (by_length) item0 = blk_first[i];
+    if (by_length && n_blk > kPlanFewBlocks) {
+      item0 = blk_first[i];
+    } else if (by_length) {
+      item0 = 0;
+      for (int j = 0; j < n_blk; ++j) item0 += items_before(blk_key[i], i, j);
+    }
     const int slot = cs_off_s[k] + fb_s[i] - fb_s[f0];
     const int comb0 = cs_off_c[k] + fb_c[i] - fb_c[f0];
     const bool fits = S == 1 || slot + rows * S <= a.cslot_cap;
@@ -3078,7 +3097,9 @@ int hx_varlen_attn_plan(const int32_t* cu_seq_q, const int32_t* cu_seq_k,
   // Blocks of all chunks: at most one per rows_per_item rows, and one more per sequence.
   const int64_t blocks = max_q >= 2 ? total_q / geo.rows_per_item + batch : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (batch <= kPlanSmallThreads && blocks <= kPlanSmallBlocks)
+  const int64_t sizes = ceil_div(max_k, kTile), full = total_q / geo.rows_per_item;
+  const bool search_fits = sizes <= kPlanSmallThreads && sizes * full <= kPlanSmallSearch;
+  if (batch <= kPlanSmallThreads && (blocks == 0 || (blocks <= kPlanSmallBlocks && search_fits)))
     hipLaunchKernelGGL((plan_kernel<kPlanSmallThreads>), dim3(1), dim3(kPlanSmallThreads), 0, s, a);
   else
     hipLaunchKernelGGL((plan_kernel<kPlanThreads>), dim3(1), dim3(kPlanThreads), 0, s, a);

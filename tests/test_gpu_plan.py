@@ -122,3 +122,12 @@ def test_plan_lists_around_the_small_planner(device, batch, chunk):
             q_lens[at], k_lens[at] = n, n + int(rng.integers(0, 3000))
     _check(f"small planner {batch} {chunk}", q_lens, k_lens, device=device)
     _check(f"small planner {batch} {chunk} window", q_lens, k_lens, window=(9000, 0), device=device)
+
+
+@pytest.mark.parametrize("chunk,k_len", [(64, 16384), (64, 16385), (512, 16384), (512, 40000), (576, 16400),
+                                         (2048, 16384), (2048, 16385), (2048, 60000)])
+def test_plan_lists_of_chunks_in_long_sequences(device, chunk, k_len):
+    """Split sizes by the hundred: the search in one pass of 256 or 1024 threads and by
+    bisection, for up to eight blocks (one thread each) and for more."""
+    _check(f"long {chunk}@{k_len}", [chunk, 1, 100], [k_len, 700, k_len - 900], device=device)
+    _check(f"long {chunk}@{k_len} alone", [chunk], [k_len], device=device)
