@@ -86,9 +86,10 @@ class PagedQwen3Decoder:
     def _few_rows(tokens: int, dtype: torch.dtype, layer: dict[str, torch.Tensor]) -> bool:
         """Whether this layer's products go to ``ops.block_linear``: few rows, and weights it
         can read."""
-        return tokens <= FEW_ROWS and dtype in (torch.bfloat16, torch.float16) and all(
+        return (tokens <= FEW_ROWS and dtype in (torch.bfloat16, torch.float16) and all(
             w.is_contiguous() and w.dtype == dtype and w.data_ptr() % 16 == 0 and w.shape[0] % 32 == 0
             and w.shape[1] % 64 == 0 for w in (layer["qkv"], layer["o"], layer["gate_up"], layer["down"]))
+            and layer["input_norm"].data_ptr() % 16 == 0 and layer["post_norm"].data_ptr() % 16 == 0)
 
     def _fused_heads(self, logit_indices: torch.Tensor, dtype: torch.dtype) -> bool:
         """Whether the logits come from the fused heads kernel: one pass over the embedding
@@ -96,7 +97,7 @@ class PagedQwen3Decoder:
         w = self.embedding
         return (logit_indices.numel() <= 160 and dtype in (torch.bfloat16, torch.float16) and w.dtype == dtype
                 and w.shape[1] % 128 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
-                and self.final_norm.dtype == torch.float32)
+                and self.final_norm.dtype == torch.float32 and self.final_norm.is_contiguous())
 
     @torch.inference_mode()
     def forward_packed(self, input_ids: torch.Tensor, cache: PackedBatchCache, *,

@@ -71,3 +71,29 @@ def test_greedy_heads_match_logits_argmax(device):
     chosen = logits.gather(1, picks.unsqueeze(1))[:, 0]
     # the kernel's pick is the argmax up to one bf16 rounding of the logits
     assert ((top - chosen) <= 2 * 2.0 ** -7 * top.abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("counts", [[1, 2], [1, 30]])
+def test_norm_weights_of_any_layout(device, counts):
+    """Norm weights that are slices of a flat buffer (4-byte aligned) and a strided final norm:
+    the same values, read by the general steps where the fused ones cannot."""
+    say("decoder norm layouts", counts)
+    config = Qwen3Config(vocab_size=640, context_length=512, hidden_size=256, n_layers=2, hidden_dim=512,
+                         dtype=torch.bfloat16)
+    model = PagedQwen3Decoder(config, device, seed=6, std=0.05)
+    ids = torch.randint(0, 640, (1, sum(counts)), generator=torch.Generator(device=device).manual_seed(7),
+                        device=device)
+    logits = []
+    for moved in (False, True):
+        if moved:
+            for layer in model.layers:
+                for name in ("input_norm", "post_norm"):
+                    layer[name] = torch.cat((layer[name][:1], layer[name]))[1:]
+            model.final_norm = model.final_norm.repeat_interleave(2)[::2]
+        pool = KVPagePool(config, 4, device=device)
+        batch = PackedBatchCache([PagedKVCache(pool, config.context_length) for _ in counts])
+        batch.prepare_packed(counts)
+        logits.append(model.forward_packed(ids, batch).float())
+    torch.cuda.synchronize()
+    # products in another order of their sums, two layers: as between the sequences above
+    assert (logits[0] - logits[1]).abs().max() <= 2e-2 * max(logits[0].abs().max().item(), 1.0)
