@@ -701,14 +701,22 @@ class VarlenAttnPlan:
         self.block_table_stride = block_table_stride
         self.window = window
         # The tuned kernels (split-K decode, MFMA chunk, combine) serve head_dim 128 with
-        # 1, 2, 4 or 8 query heads per KV head; other shapes run one generic kernel that
-        # covers every row in a single launch.
+        # 1, 2, 4 or 8 query heads per KV head; other shapes run one kernel for every row and
+        # one that merges their splits.
         self.tuned = head_dim == 128 and n_kv_heads > 0 and n_q_heads % n_kv_heads == 0 \
             and n_q_heads // n_kv_heads in (1, 2, 4, 8)
         self._metadata = (cu_seq_q.contiguous(), None if cu_seq_k is None else cu_seq_k.contiguous(),
                           None if seqused_k is None else seqused_k.contiguous())
         self.ws_bytes = workspace_bytes(max(batch, 0), max_q, max_k, n_q_heads, n_kv_heads, head_dim)
-        self.workspace = torch.empty(self.ws_bytes + 256, dtype=torch.uint8, device=device)
+        try:
+            self.workspace = torch.empty(self.ws_bytes + 256, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            # Without room for fp32 partials the untuned shapes run in less (whole rows).
+            least = workspace_bytes(max(batch, 0), max_q, max_k, n_q_heads, n_kv_heads, 8)
+            if self.tuned or least >= self.ws_bytes:
+                raise
+            self.ws_bytes = least
+            self.workspace = torch.empty(self.ws_bytes + 256, dtype=torch.uint8, device=device)
         base = self.workspace.data_ptr()
         self._ws_offset = (-base) % 256
         self.ws_ptr = base + self._ws_offset
@@ -925,9 +933,9 @@ class VarlenAttnPlan:
             self.hints[2] if "combine" in phases else 0,
         )
         if not self.tuned:
-            # The generic kernel covers every row in one launch: it runs in the call that
-            # holds the decode phase, or in the chunk phase of a tick without decode rows,
-            # never twice for one layer.
+            # The any-head_dim kernel covers every row in one launch and merges in the next:
+            # both run in the call that holds the decode phase, or in the chunk phase of a
+            # tick without decode rows, never twice for one layer.
             once = "decode" in phases or ("chunk" in phases and self.hints[0] == 0)
             hints = (self.hints[0], self.hints[1], hints[2]) if once else (0, 0, hints[2])
         common = (
@@ -1042,7 +1050,7 @@ def run_overlapped(plan: "VarlenAttnPlan", query: torch.Tensor, k_cache: torch.T
     side stream before the chunk launch (work that must also overlap the decode rows);
     its return value is returned last, and any tensors in it are marked as used by the
     current stream. Falls back to ``plan.run`` when one kind of row is absent, and for
-    shapes the generic kernel serves (it covers every row in one launch)."""
+    shapes the any-head_dim kernel serves (it covers every row in one launch)."""
     dec, pf, _ = plan.hints
     has_chunk = pf != 0 and plan.max_q >= 2
     if dec == 0 or (not has_chunk and side_first is None) or not plan.tuned:

@@ -134,8 +134,10 @@ int hx_kv_gather(const void* pool, int32_t num_pool_pages, int32_t page_size,
  * run a bf16/fp16 MFMA kernel. Every other shape runs one MFMA kernel for all rows over
  * the same kind of splits, blocks of 64 (row, query head) pairs of a KV head sharing each
  * 64-key K/V tile through LDS, with fp32 scores, P and partials, and a deterministic
- * combine. In a workspace below the size stated here but not below that of
- * the same heads at head_dim 128, it runs without splits.
+ * combine. Its fp32 partials
+ * make hx_varlen_attn_workspace_bytes up to 4 times (head_dim 256) what 16-bit ones of 128
+ * dims take. In a smaller workspace, but not below the size for the same heads at head_dim
+ * 8, it runs without splits, each row or block of rows whole.
  *
  * The workspace (size from hx_varlen_attn_workspace_bytes, 256-byte aligned) holds
  * the work plan and the split-K partials. hx_varlen_attn_plan writes the plan from
@@ -153,7 +155,9 @@ size_t hx_varlen_attn_workspace_bytes(int32_t batch, int32_t max_q, int32_t max_
                                       int32_t head_dim);
 
 /* Host-side item counts for known lengths (q_lens[b] = n_b, k_lens[b] = L_b, HOST
- * arrays); mirrors the device planner exactly. Returns 0 or HX_E_INVALID_ARG. */
+ * arrays); mirrors the device planner exactly for the tuned shapes (head_dim 128, 1, 2, 4 or
+ * 8 query heads per KV head). The any-head_dim kernel is planned in blocks of its own, and
+ * its runs take from the hints only whether they are 0. Returns 0 or HX_E_INVALID_ARG. */
 int hx_varlen_attn_count_items(const int32_t* q_lens, const int32_t* k_lens, int32_t batch,
                                int32_t n_q_heads, int32_t n_kv_heads,
                                int32_t window_left, int32_t window_right,
@@ -391,7 +395,7 @@ size_t hx_varlen_attn_error_word_offset(void);
  * address is looked up once per GPU, at that GPU's first call (make that first call
  * outside graph capture), with the stream's GPU current.
  *   - A shape whose workspace (hx_varlen_attn_workspace_bytes; for shapes served by the
- *     any-head_dim kernel, that of the same heads at head_dim 128) exceeds the array
+ *     any-head_dim kernel, that of the same heads at head_dim 8) exceeds the array
  *     returns HX_E_TOO_LARGE before any launch. Decode ticks of up to ~15000 256-key
  *     splits fit, and so do the mixed and long-context ticks of the Qwen3-4B
  *     workloads (about 71-100 MiB).

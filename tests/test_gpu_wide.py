@@ -201,3 +201,25 @@ def test_infinite_and_nan_values(device, hq, hkv, d, dtype):
         assert np.abs(lse.cpu().numpy() - lse0.cpu().numpy())[same].max() < 1e-4
         v_flat.copy_(keep)
         k_flat.copy_(k_keep)
+
+
+def test_workspace_without_room_for_fp32_partials(device, monkeypatch):
+    """A plan whose full workspace cannot be allocated takes the smaller one and runs whole
+    rows; a tuned shape, which has no smaller one, raises."""
+    say("wide workspace fallback")
+    tick = _tick([min(n, 3) for n in Q_LENS], K_LENS, 4, 1, 256, torch.bfloat16, device, 900)
+    tuned = _tick([1, 5], [300, 40], 8, 2, 128, torch.bfloat16, device, 901)
+    ref, _ = tick.oracle()
+    full = {ops.workspace_bytes(t.w.batch, t.w.max_q, t.w.max_k, t.w.n_q_heads, t.w.n_kv_heads, t.w.head_dim) + 256
+            for t in (tick, tuned)}
+    empty = torch.empty
+
+    def no_room(*args, **kwargs):
+        if args and args[0] in full:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", no_room)
+    compare(tick.attend(exact_grid=True), ref, what="wide workspace fallback")
+    with pytest.raises(torch.OutOfMemoryError):
+        tuned.plan()
