@@ -2951,7 +2951,9 @@ int launch_wide(const RunArgs& a, const WideShape& ws, hipStream_t s) {
   else if (ws.head_dim <= 96) hipLaunchKernelGGL((wide_kernel<T, 96>), grid, block, 0, s, a, ws, wgs);
   else if (ws.head_dim <= 128) hipLaunchKernelGGL((wide_kernel<T, 128>), grid, block, 0, s, a, ws, wgs);
   else hipLaunchKernelGGL((wide_kernel<T, 256>), grid, block, 0, s, a, ws, wgs);
-  if (ws.lists && ws.max_comb > 0) {
+  // Up to max_k = kSplit nothing is split (a chunk block has kMinSplitTiles tiles at most).
+  static_assert(kMinSplitTiles * kTile >= kSplit, "a block of kSplit keys stays whole");
+  if (ws.lists && ws.max_comb > 0 && a.max_k > kSplit) {
     const int64_t merges = ws.max_comb * a.hkv;
     const int cw = (int)(merges < kWideWGs ? merges : kWideWGs);
     hipLaunchKernelGGL((wide_combine_kernel<T>), dim3((unsigned)cw), block, 0, s, a, ws, cw);
