@@ -244,9 +244,11 @@ __global__ __launch_bounds__(kLgThreads) void logits_argmax_kernel(
 // The same product for many logit rows, where reading fragments from LDS costs more than the
 // weight stream: 8 waves x 5 MFMA tiles of vocab rows, so that an x fragment read feeds five
 // MFMAs instead of two, in one workgroup per CU (HBM and MFMA bound in turn: 129 rows take
-// 177 us, 4.4 TB/s of weights; 64 rows and fewer are faster above). The first pass over a
-// table not read before loses 7 us at 129 rows (250 us against 243), a repeated one gains
-// 15. Weights and x go from memory straight into LDS, 32 hidden elements at a time, into three buffers used in turn: two chunks are in
+// 177 us, 4.4 TB/s of weights; 64 rows and fewer are faster above). It reads the table in 64-byte
+// pieces of 5-KiB rows all over it, and that pattern suffers from dirty lines that earlier
+// writes left in the memory-side cache: right after 778 MB of zeros, or a table's own filling,
+// a call takes 247 us here and 222 above, also after 20 ms of idling; the next one 203 and 220.
+// Weights and x go from memory straight into LDS, 32 hidden elements at a time, into three buffers used in turn: two chunks are in
 // flight while one is consumed, and a chunk costs one wait and one barrier.
 //
 // LDS rows are 64 bytes; the 16-byte piece at position p of row r is piece p ^ ((r >> 2) & 3),
@@ -421,10 +423,13 @@ LogitsLayout logits_layout(int64_t n_rows, int64_t vocab, int32_t hidden) {
 
 // From kLtMinTiles row tiles on, and where its 640-row workgroups fill at least three quarters
 // of the rounds of one per CU that they take, the wide kernel. A call at 151936 x 2560 bf16
-// (norm, product, reduce; in us, with the logits written): 80 rows 168 (179) there against 160
-// (180) here, 100 rows 174 (186) against 180 (197), 129 rows 187 (199) against 200 (216), 160
-// rows 193 (207) against 213 (229). Row offsets within a workgroup are 32-bit: ld_emb below 2^20.
-constexpr int kLtMinTiles = 7;
+// (norm, product, reduce; in us, with the logits written), after products of 1152 rows as in a
+// tick, whose writes cost it: 112 rows 195 (199) there against 184 (203) here, 128 rows 199
+// (203) against 195 (210), 129 rows 206 (211) against 206 (221), 160 rows 209 (214) against 220
+// (234). On its own: 112 rows 174 (187) against 178 (196), 129 rows 185 (197) against 197
+// (214), 160 rows 190 (202) against 210 (225). Row offsets within a workgroup are 32-bit:
+// ld_emb below 2^20.
+constexpr int kLtMinTiles = 9;
 
 // Launches one group's product; returns its workgroups over the vocab (partial keys a row).
 template <typename T, int NT>

@@ -77,9 +77,10 @@ def test_matches_oracle(device, dtype, picks):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("picks", [97, 113, 129, 160])
 def test_many_rows_over_640_row_vocab_tiles(device, picks, dtype):
-    """The kernel for seven and more row tiles, which needs a vocab that fills the chip: 199
-    workgroups of 640 rows, the last of them 29 rows, hidden of five buffer turns and a
-    rest. Against fp32 products of the same normalised rows, every logit and pick."""
+    """Around the kernel for nine and more row tiles (129 rows on), which needs a vocab that
+    fills the chip: 199 workgroups of 640 rows, the last of them 29 rows, hidden of five
+    buffer turns and a rest. Every logit and pick against the few-row kernel's and against
+    float64 products of the same normalised rows."""
     say("logits many rows", picks, dtype)
     hidden, vocab = 512, 198 * 640 + 29
     x, w, emb, idx = _inputs(device, 200, hidden, vocab, picks, seed=picks, std=0.03)
@@ -94,6 +95,14 @@ def test_many_rows_over_640_row_vocab_tiles(device, picks, dtype):
     assert ((got - want).abs() <= ulp * want.abs() + 1e-5).all()
     assert (got != want).float().mean() < 2e-2
     assert torch.equal(res.token_ids, got.argmax(dim=-1)) and torch.equal(res.max_logits, got.max(dim=-1).values)
+    # float64 products of rows normalised and rounded as the reference does, within the bound
+    # of the oracle's test above: the logit's rounding, and an element of the normalised row
+    # that rounds one step apart, times the largest weight
+    rows = x[idx].float()
+    rows = (rows * torch.rsqrt(rows.pow(2).mean(-1, keepdim=True) + 1e-6) * w).to(dtype).double()
+    exact = torch.cat([rows @ part.double().t() for part in emb.split(16384)], dim=1)
+    moved = ulp * rows.abs().amax(dim=1, keepdim=True) * emb.double().abs().max()
+    assert ((got.double() - exact).abs() <= 2 * ulp * exact.abs() + moved).all()
 
 
 def test_ties_and_planted_winners(device):
