@@ -86,7 +86,7 @@ def test_c5_attention_layer_matches_oracle(device):
     batch.advance_packed()
 
 
-def test_c5_full_forward_greedy_properties(device):
+def test_c5_full_forward_greedy_properties(device, monkeypatch):
     from helios_amd.decoder import PagedQwen3Decoder
 
     say("c5 36-layer forward, greedy heads")
@@ -98,7 +98,10 @@ def test_c5_full_forward_greedy_properties(device):
                               generator=torch.Generator(device=device).manual_seed(52), device=device)
     batch = PackedBatchCache(caches)
     outs = []
-    for greedy in (True, False):
+    for greedy, fused in ((True, True), (False, False), (False, True)):
+        monkeypatch.undo()
+        if not fused:  # the library's logits: an independent lm_head
+            monkeypatch.setattr(PagedQwen3Decoder, "_fused_heads", lambda *a: False)
         batch.prepare_packed(counts)
         outs.append(model.forward_packed(input_ids, batch, greedy=greedy))
         torch.cuda.synchronize()
@@ -119,3 +122,10 @@ def test_c5_full_forward_greedy_properties(device):
     apart = (top2[:, 0] - top2[:, 1]) > 2 * ulp
     say("clear winners", int(apart.sum()), "of", len(counts))
     assert torch.equal(ids[apart], logits.argmax(dim=-1)[apart])
+    # The fused logits: the same products in another order of their sums, and elements of the
+    # normalised row (of rms 1, 2^-7 of up to 8) that round a step apart, times the largest weight.
+    fused_logits = outs[2].float().cpu()
+    moved = 2.0 ** -7 * 8 * model.embedding.abs().max().item()
+    assert bool(((fused_logits - logits).abs() <= 2 * 2.0 ** -7 * logits.abs() + moved).all())
+    assert float((fused_logits != logits).float().mean()) < 5e-2
+    assert torch.equal(ids, fused_logits.argmax(dim=-1))

@@ -49,13 +49,18 @@ def test_packed_forward_matches_reference_sequence(device):
     assert torch.equal(pools[0], pools[1])  # values are appended bit-exactly by both paths
 
 
-def test_greedy_heads_match_logits_argmax(device):
+def test_greedy_heads_match_logits_argmax(device, monkeypatch):
+    """The fused heads' ids and logits against the library's logits (final norm, product with
+    the embedding) of the same tick."""
     say("decoder greedy heads")
     config = Qwen3Config(vocab_size=1000, context_length=4096, hidden_size=256, n_layers=2,
                          hidden_dim=512, dtype=torch.bfloat16)
     model = PagedQwen3Decoder(config, device, seed=2, std=0.05)
     outs = []
-    for greedy in (False, True):
+    for greedy, fused in ((False, False), (True, True), (False, True)):
+        monkeypatch.undo()
+        if not fused:
+            monkeypatch.setattr(PagedQwen3Decoder, "_fused_heads", lambda *a: False)
         pool = KVPagePool(config, 8, device=device)
         caches = [PagedKVCache(pool, config.context_length) for _ in range(3)]
         batch = PackedBatchCache(caches)
@@ -71,6 +76,12 @@ def test_greedy_heads_match_logits_argmax(device):
     chosen = logits.gather(1, picks.unsqueeze(1))[:, 0]
     # the kernel's pick is the argmax up to one bf16 rounding of the logits
     assert ((top - chosen) <= 2 * 2.0 ** -7 * top.abs() + 1e-4).all()
+    # The same bf16 products in another order of their fp32 sums: one rounding step apart. An
+    # element of the normalised row (of rms 1) may round a step (2^-7 of itself) apart as well.
+    fused_logits = outs[2].float().cpu()
+    moved = 2.0 ** -7 * 4 * model.embedding.abs().max().item()
+    assert ((fused_logits - logits).abs() <= 2 * 2.0 ** -7 * logits.abs() + moved).all()
+    assert torch.equal(picks, fused_logits.argmax(dim=-1))
 
 
 @pytest.mark.parametrize("counts", [[1, 2], [1, 30]])
