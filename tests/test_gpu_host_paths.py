@@ -47,7 +47,24 @@ def test_short_host_paths_give_the_bits_of_the_general_ones(device, monkeypatch)
         return out.clone(), out.stride(), pool.storage.clone()
 
     for projected in (False, True):
-        short = tick(projected)
+        taken = []
+
+        def watch(m, owner, name):
+            inner = getattr(owner, name)
+
+            def call(*a):
+                out = inner(*a)
+                taken.append((name, out is not None))
+                return out
+            m.setattr(owner, name, call)
+
+        with monkeypatch.context() as m:
+            watch(m, ops.VarlenAttnPlan, "append_attend")
+            watch(m, ops.VarlenAttnPlan, "attend_rows")
+            watch(m, ops, "qk_norm_rope_append_packed")
+            short = tick(projected)
+        assert taken == ([("qk_norm_rope_append_packed", True), ("attend_rows", True)] if projected
+                         else [("append_attend", True)])
         with monkeypatch.context() as m:
             m.setattr(ops.VarlenAttnPlan, "append_attend", lambda *a: None)
             m.setattr(ops.VarlenAttnPlan, "attend_rows", lambda *a: None)
