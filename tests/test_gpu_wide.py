@@ -89,7 +89,7 @@ def test_wide_without_work_lists(device, hq, hkv, d, monkeypatch):
     tick = _tick([min(n, 3) for n in Q_LENS], K_LENS, hq, hkv, d, torch.bfloat16, device, 500 + d)
     ref, ref_lse = tick.oracle()
     sized = ops.workspace_bytes
-    least = sized(tick.w.batch, tick.w.max_q, tick.w.max_k, hq, hkv, 128)
+    least = sized(tick.w.batch, tick.w.max_q, tick.w.max_k, hq, hkv, 8)
     assert least < sized(tick.w.batch, tick.w.max_q, tick.w.max_k, hq, hkv, d)
     monkeypatch.setattr(ops, "workspace_bytes", lambda *a: least)
     out, lse = tick.attend(exact_grid=True, return_lse=True)
@@ -223,3 +223,28 @@ def test_workspace_without_room_for_fp32_partials(device, monkeypatch):
     compare(tick.attend(exact_grid=True), ref, what="wide workspace fallback")
     with pytest.raises(torch.OutOfMemoryError):
         tuned.plan()
+
+
+def test_wide_items_of_more_than_64_pages(device, monkeypatch):
+    """A workgroup holds 64 page ids at a time: items of 16384 keys and around it, and of 33000
+    (three fetches), on shuffled pages. Whole decode rows and a chunk without work lists, and
+    a chunk of so many blocks that none is split."""
+    say("wide many pages, whole rows")
+    tick = _tick([1, 1, 1, 1, 3], [16384, 16385, 16640, 33000, 32769], 1, 1, 136, torch.bfloat16, device, 950)
+    sized = ops.workspace_bytes
+    least = sized(tick.w.batch, tick.w.max_q, tick.w.max_k, 1, 1, 8)
+    assert least < sized(tick.w.batch, tick.w.max_q, tick.w.max_k, 1, 1, 136)
+    ref, ref_lse = tick.oracle()
+    with monkeypatch.context() as m:
+        m.setattr(ops, "workspace_bytes", lambda *a: least)
+        out, lse = tick.attend(exact_grid=True, return_lse=True)
+    compare(out, ref, what="wide many pages, whole rows")
+    assert np.abs(lse.cpu().numpy() - ref_lse).max() < 1e-4
+
+    say("wide many pages, unsplit chunk")
+    # 64 heads on one: a block a row, so 520 rows are 520 items, and 512 are not split
+    tick = _tick([520, 1], [17000, 16641], 64, 1, 8, torch.bfloat16, device, 951)
+    rows = {0: [0, 1, 255, 518, 519], 1: [0]}
+    ref, _ = tick.oracle(rows=rows)
+    out = tick.attend(exact_grid=True)
+    compare(out, ref, what="wide many pages, unsplit chunk", rows=np.array(rows[0] + [520]))
