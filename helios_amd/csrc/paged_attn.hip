@@ -586,7 +586,7 @@ constexpr int kPlanSearchWork = 1 << 16;  // candidates x blocks evaluated in on
 constexpr int kPlanSortBlocks = 256;
 // Ticks of at most 256 sequences and 96 blocks take 256 threads: every pass ends in barriers
 // and per-wave totals, and four waves get through them sooner than sixteen (64 decode rows
-// 5.6 -> 3.9 us; 14, 64 and 76 blocks 12.3 -> 9.4, 9.7 -> 7.7 and 13.3 -> 12.0 us; 126 blocks
+// 5.6 -> 4.0 us; 14, 64 and 76 blocks 12.3 -> 9.5, 9.7 -> 7.7 and 13.3 -> 12.1 us; 126 blocks
 // would be slower).
 // The split-size search has to fit them as well, one size (of up to max_k / 64) a thread and
 // 32 blocks' counts each. Beyond, 1024 threads are sooner: 32/8 heads, 1024 rows at 32768 keys
@@ -2203,10 +2203,10 @@ __global__ __launch_bounds__(kChunkThreads, 2) void chunk_pair_kernel(RunArgs a0
 // below the error of the exp, and 2^-37 absolute of a smaller one (p is scaled by 2^12). Two
 // bf16 (17 bits) showed where values cancel: 100 keys against 100 with weights 1/2000 apart
 // came out 0.57 % off instead of 0.18 %, of which the output's rounding is 0.17 %. The third
-// costs chunks 5-13 % and decode rows, whose 16 keys fill half an operand, nothing. The splits'
+// costs chunks 5-17 % and decode rows, whose 16 keys fill half an operand, nothing. The splits'
 // partial results stay in fp32. q . k is exact products in fp32 sums.
 // Bound by latency at these sizes. 24 decode rows of 200-2048 keys and chunks of 512 and
-// 333 rows, 16/4 heads, d = 64: 18.6 us and 4.8 us for the merge; scores and P V on the VALU,
+// 333 rows, 16/4 heads, d = 64: 19.8 us and 5.0 us for the merge; scores and P V on the VALU,
 // 16 units a workgroup and no splits, took 284 us. Two tiles in flight instead of one gained
 // nothing. Workgroups per CU by padded head dim (the launch bounds): at 128 a third and at 256 a
 // second one (chunks of 600 rows at 256: 107.6 -> 89.6 us a call; at 96 a third lost 5 %).

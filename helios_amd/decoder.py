@@ -50,6 +50,11 @@ def _apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, positions
 # Ticks of at most this many rows run their products through ops.block_linear: a layer's four
 # products and the steps between them take 62-71 us that way and 102 us on hipBLASLt at up to
 # 16 rows (one MFMA row tile); at 17-32 rows hipBLASLt's take 77-82 us, a second row tile 88-94.
+# That is hidden 2560, ffn 9728, 32/8 heads of 128. At other widths, 1 / 8 / 16 rows against
+# hipBLASLt: 256 and 768 12 / 14 / 15 us against 28 / 30 / 30; 1024 and 3072 20 / 21 / 24 against
+# 39 / 40 / 40; 2048 and 6144 37 / 40 / 44 against 52; 4096 and 12288 85 / 88 / 100 against 99 /
+# 100 / 101; 5120 and 17408 165 / 177 / 207 against 243 / 248 / 252; 8192 and 28672 304 / 314 /
+# 356 against 346 / 347 / 352.
 FEW_ROWS = 16
 
 

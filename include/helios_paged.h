@@ -143,7 +143,8 @@ int hx_kv_gather(const void* pool, int32_t num_pool_pages, int32_t page_size,
  * the work plan and the split-K partials. hx_varlen_attn_plan writes the plan from
  * the metadata; hx_varlen_attn_run consumes it and may be called any number of
  * times (e.g. once per layer) while cu_seq_q / cu_seq_k / seqused_k and the scalar
- * shape arguments are unchanged. hx_varlen_attn = plan + run.
+ * shape arguments are unchanged. Runs write the split partials: those that share a
+ * workspace must be ordered, as calls on one stream are. hx_varlen_attn = plan + run.
  *
  * decode_items_hint / prefill_items_hint size the launch grids. Pass -1 to use the
  * bound derived from (batch, max_q, max_k); a caller that knows the host-side

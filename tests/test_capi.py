@@ -45,7 +45,7 @@ def test_abi_version_and_strerror():
 def test_workspace_bytes_supported_shapes():
     lib = _capi.lib()
     assert lib.hx_varlen_attn_workspace_bytes(64, 1, 4097, 32, 8, 128) > 0
-    # any head_dim that is a multiple of 8 up to 256, any group size (the generic kernel)
+    # any head_dim that is a multiple of 8 up to 256, any group size (the any-head_dim kernel)
     for hq, hkv, d in ((32, 8, 64), (48, 8, 128), (2, 1, 8), (64, 1, 256), (12, 4, 96)):
         assert lib.hx_varlen_attn_workspace_bytes(64, 1, 4097, hq, hkv, d) > 0, (hq, hkv, d)
     for d in (0, 4, 12, 130, 264):

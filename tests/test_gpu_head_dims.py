@@ -1,4 +1,4 @@
-"""Attention at head dims and group sizes other than Qwen3-4B's (the generic kernel),
+"""Attention at head dims and group sizes other than Qwen3-4B's (the any-head_dim kernel),
 against the float64 oracle, and the reference's own GPU test of the paged boundary
 (tests/test_paged_attention.py:240-312) at its own tiny shape through the class-level
 drop-in: head_dim 8, 2 query heads on 1 KV head, fp16 and bf16, a 2-token prefill of two

@@ -5,7 +5,7 @@
   launch, or the append kernel when the call launches no work that writes them (a
   decode-phase call on a chunk-only tick, a combine-only call). Checked bit for bit
   against the rows given.
-* On shapes the generic kernel serves, ``run_overlapped`` gives the bits of ``run``.
+* On shapes the any-head_dim kernel serves, ``run_overlapped`` gives the bits of ``run``.
 """
 
 from __future__ import annotations
@@ -54,7 +54,7 @@ def test_append_is_written_by_every_phase_set(device, name, phases):
 
 
 def test_generic_shape_overlapped_matches_run(device):
-    """head_dim 64 (generic kernel), decode rows and chunks on two streams."""
+    """head_dim 64 (any-head_dim kernel), decode rows and chunks on two streams."""
     w = synth.small_mixed(64, n_q_heads=8, n_kv_heads=2, head_dim=64, batch=6)
     assert 1 in w.q_lens and max(w.q_lens) > 1
     tick = DeviceTick(w, torch.bfloat16, device)

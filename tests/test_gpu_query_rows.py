@@ -3,7 +3,7 @@ query_rows=...)``, ``hx_varlen_attn_run_rows``).
 
 The shared-prefix cascade runs its prefix levels over member rows that repeat the tick's
 decode rows, and reads them in place through such a map. The result must be the run on
-the gathered queries, bit for bit, for decode rows, chunk rows and the generic kernel's
+the gathered queries, bit for bit, for decode rows, chunk rows and the any-head_dim kernel's
 shapes; a map entry outside the query tensor raises its error-word bit and reads row 0.
 """
 

@@ -1,8 +1,8 @@
 """Randomized mixed ticks against the float64 oracle.
 
 Each case draws, from its seed, the shapes the kernels branch on:
-- the group size: 1, 2, 4 or 8 (tuned at head_dim 128), or 3 (the generic kernel);
-- head_dim: 128, or 64 / 96 (the generic kernel);
+- the group size: 1, 2, 4 or 8 (tuned at head_dim 128), or 3 (the any-head_dim kernel);
+- head_dim: 128, or 64 / 96 (the any-head_dim kernel);
 - dtype (bf16 or fp16), page size (256 or 512) and the attention window;
 - the tick's mix: decode rows, short and long chunks, rows crossing page boundaries.
 
